@@ -217,9 +217,17 @@ struct Loader {
   // loaded lane by lane with bounds checks.  INB (with ALIGNED): the kernel
   // has proved that every tile it loads lies inside the tensor, so neither
   // the tile base nor a lane's offset selects the zero page.
-  template <bool ALIGNED, bool INB = false>
+  //
+  // CLAMP (with INB; 1 = rows, 2 = columns): the tile's origin is inside but
+  // it may straddle the tensor's end in that dimension, one that the program
+  // id indexes (M or N of a product).  Lanes past the end read the last row or
+  // 16-byte chunk instead of zeros: they feed only result rows or columns that
+  // are past the end too and are never stored.  The clamp sits in the lane
+  // offsets, which do not depend on the loop, so it costs nothing per step.
+  template <bool ALIGNED, bool INB = false, int CLAMP = 0>
   static __device__ __forceinline__ Src prep(const gl<bf16>& g, int b, int d, int row0, int col0) {
     static_assert(ALIGNED || !INB, "the in-bounds form is a case of the aligned one");
+    static_assert(INB || CLAMP == 0, "clamped lanes are a case of the in-bounds form");
     const bool bd_ok = (unsigned)b < (unsigned)g.b && (unsigned)d < (unsigned)g.d;
     const bf16* bd = g.data + (long long)b * g.sb + (long long)d * g.sd;
     if (ALIGNED) {
@@ -233,13 +241,15 @@ struct Loader {
   }
 
   // Issue this wave's j-th DMA instruction of the tile.
-  template <bool ALIGNED, bool INB = false>
+  template <bool ALIGNED, bool INB = false, int CLAMP = 0>
   static __device__ __forceinline__ void issue(int j, char* tile_base, const gl<bf16>& g, const Src& s, int wave) {
     int row, c;
     place(wave, j, row, c);
     const unsigned dst = lds_addr(tile_base + (wave + j * NW) * 1024);
     if (ALIGNED) {
-      const unsigned voff = (INB || s.inb) ? (unsigned)(row * (int)g.sr + c * 8) * 2u : 0u;
+      if (CLAMP == 1) row = min(row, g.r - 1 - s.row0);
+      const int col = CLAMP == 2 ? min(c * 8, g.c - 8 - s.col0) : c * 8;
+      const unsigned voff = (INB || s.inb) ? (unsigned)(row * (int)g.sr + col) * 2u : 0u;
       dma16_s(s.base, voff, dst);
       return;
     }
@@ -253,17 +263,23 @@ struct Loader {
     }
   }
 
-  template <bool ALIGNED, bool INB = false>
+  template <bool ALIGNED, bool INB = false, int CLAMP = 0>
   static __device__ __forceinline__ void load(char* tile_base, const gl<bf16>& g, int b, int d, int row0,
                                               int col0, int wave) {
-    const Src src = prep<ALIGNED, INB>(g, b, d, row0, col0);
+    const Src src = prep<ALIGNED, INB, CLAMP>(g, b, d, row0, col0);
 #pragma unroll
-    for (int j = 0; j < INSTR_PER_WAVE; ++j) issue<ALIGNED, INB>(j, tile_base, g, src, wave);
+    for (int j = 0; j < INSTR_PER_WAVE; ++j) issue<ALIGNED, INB, CLAMP>(j, tile_base, g, src, wave);
   }
 
   // Whether `g` qualifies for the kernel's ALIGNED specialisation.
   static __device__ __forceinline__ bool aligned(const gl<bf16>& g) {
     return g.r % Tile::ROWS == 0 && g.c % Tile::COLS == 0 && (long long)Tile::ROWS * g.sr < (1ll << 30);
+  }
+
+  // Whether `g` suits the clamped form: whole 16-byte chunks per row, and a
+  // row pitch that fits the 32-bit lane offsets.
+  static __device__ __forceinline__ bool clampable(const gl<bf16>& g) {
+    return g.c % 8 == 0 && (long long)Tile::ROWS * g.sr < (1ll << 30);
   }
 };
 
@@ -290,9 +306,10 @@ struct VecLoader {
   }
 };
 
-template <bool B>
+// Selects a kernel's body: value = the aligned form, edge = its clamped variant.
+template <bool B, bool EDGE = false>
 struct bool_tag {
-  static constexpr bool value = B;
+  static constexpr bool value = B, edge = EDGE;
 };
 
 // Wait until at most N of this wave's vector-memory instructions are

@@ -275,6 +275,10 @@ TARGETS: Dict[str, dict] = {
     "gemm_128_splitk_k64_b7sw": {"dma_spread_whole": True},
     "gemm_128_splitk_k32_b14sw": {"dma_spread_whole": True},
 }
+# the products that api.gemm launches run ragged extents in the clamped body
+for _name in ("gemm_256_k64", "gemm_256x128", "gemm_128_k64", "gemm_128x64_k64", "gemm_128x32_k64",
+              "gemm_128_splitk_k64_b7"):
+    TARGETS[_name] = {**TARGETS.get(_name, {}), "clamp_edges": True}
 # the lazy softmax's row sums on the matrix core (CDNA4Target.rowsum_mfma; config 5 within 0.3-0.7%
 # of the default, the config-4 ping-pong 5% slower)
 for _base in ("mha_d128", "mha_d64_causal"):

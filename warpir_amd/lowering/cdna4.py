@@ -169,6 +169,14 @@ class CDNA4Target:
     # rings whose wait leaves the newest batch in flight (a deeper ring on
     # the operand loaded last), where those loads have a step more to land.
     dma_spread_whole: bool = False
+    # Ring-buffered products: a third body for extents that are no multiples of
+    # the tile.  It is the in-bounds one with the program-id dimension of each
+    # tile clamped in its lane offsets (wir::Loader's CLAMP) and one checked
+    # copy of the loop body for a reduction extent that cuts the last tile;
+    # the checked body (a bounds test and a 64-bit select per lane and DMA, one
+    # loop copy with run-time slots) is left to extents that fit neither.
+    # gemm_256_k64 at 3000x4104x4040: 134.7 us in the checked body, 97.9 in this.
+    clamp_edges: bool = False
     # Element-wise register-tile ops that directly precede an MMA emitted from
     # register operands (hoisted fragments, or a bf16 register A) and that the
     # MMA does not depend on run inside that MMA's MFMA stream, one group of
@@ -247,6 +255,8 @@ class CDNA4Lowerer:
         self._ws_producer_streams = self._ws_streams(kernel) if self._ws else set()
         if self._ws and self._ws_producer_streams is None:
             self._ws = False
+        self._edge = (self.target.clamp_edges and not self._ws and not self.target.persistent
+                      and _buffer_form(kernel))
         if self.target.lazy_softmax:
             for loop in _walk(kernel.body):
                 if isinstance(loop, ForOp):
@@ -451,6 +461,7 @@ class CDNA4Lowerer:
         self._fused_loads: Dict[int, List[Op]] = {}
         self._fused_ids: set = set()
         self._var_override: Dict[str, str] = {}  # resolved value name -> C++ variable
+        self._edge = False                        # buffer-form loads carry their clamp (WIR_EDGE body)
         self._ws = False                          # warp-specialised form (producer / consumer waves)
         self._softmax_fused: Dict[int, object] = {}  # id(op) -> fused lazy-softmax plan, or "skip"
         self._slot_work: Dict[int, tuple] = {}       # id(MMA) -> (moved ops, register groups, slots form)
@@ -1090,7 +1101,7 @@ class CDNA4Lowerer:
             src = op.source
             sub = src.type.sub_tile_type
             b, d, rt, ct = (self._int(c) for c in op.coords)
-            call = f"{self._load_call(op, 'load<WIR_AL, WIR_INB>(', ptr, key)});"
+            call = f"{self._load_call(op, f'load<WIR_AL, WIR_INB{self._clamp_arg(op)}>(', ptr, key)});"
             if self._ws:
                 who = self._ws_issuer(op.buf.name) if isinstance(op, TMALoadBufOp) else "wir_producer"
                 w(f"{pad}if ({who}) {call}")
@@ -1134,14 +1145,15 @@ class CDNA4Lowerer:
                     sub = ld.source.type.sub_tile_type
                     bb, dd, rt, ct = (self._int(c) for c in ld.coords)
                     self._aligned_checks.add((self.stile(lkey), _cname(ld.source.name)[2:]))
-                    w(f"{pad}const auto src{n_ld}_ = {loader}::prep<WIR_AL, WIR_INB>({g}, {bb}, {dd}, ({rt}) * {sub.rows}, "
+                    cl = self._clamp_arg(ld)
+                    w(f"{pad}const auto src{n_ld}_ = {loader}::prep<WIR_AL, WIR_INB{cl}>({g}, {bb}, {dd}, ({rt}) * {sub.rows}, "
                       f"({ct}) * {sub.cols});")
                     if self._ws and self.resolve(ld.buf.name) in self._ws_producer_streams:
-                        pcalls.append(f"if (q >= {ptotal} && q < {ptotal + n}) {loader}::issue<WIR_AL, WIR_INB>(q - {ptotal}, "
+                        pcalls.append(f"if (q >= {ptotal} && q < {ptotal + n}) {loader}::issue<WIR_AL, WIR_INB{cl}>(q - {ptotal}, "
                                       f"{lptr}, {g}, src{n_ld}_, wir_wave);")
                         ptotal += n
                         continue
-                    calls.append(f"if (q >= {total} && q < {total + n}) {loader}::issue<WIR_AL, WIR_INB>(q - {total}, "
+                    calls.append(f"if (q >= {total} && q < {total + n}) {loader}::issue<WIR_AL, WIR_INB{cl}>(q - {total}, "
                                  f"{lptr}, {g}, src{n_ld}_, wir_wave);")
                     total += n
                 if self._ws:
@@ -1280,6 +1292,14 @@ class CDNA4Lowerer:
             self._emit_for(op, out, depth)
             return
         raise LoweringError(f"no CDNA4 lowering for {type(op).__name__}")
+
+    def _clamp_arg(self, op) -> str:
+        """Template argument of a buffer-form tile load: the dimension that a
+        program id indexes, clamped in the WIR_EDGE body (``wir::Loader``)."""
+        if not self._edge or not isinstance(op, TMALoadBufOp):
+            return ""
+        dims = [k for k, c in ((1, op.coords[2]), (2, op.coords[3])) if isinstance(c, Value) and c.name in _GRID]
+        return f", WIR_EDGE ? {dims[0]} : 0" if len(dims) == 1 else ""
 
     def _load_call(self, op, fn: str, ptr: str, key: str) -> str:
         src = op.source
@@ -1521,10 +1541,17 @@ class CDNA4Lowerer:
             out.append(f"{pad}}}")
             return
         base = f"wir_base_{iv[2:]}"
+        tail = self._checked_tail(op)
+        full = stop
+        if tail:
+            # the clamped body runs the tiles that are whole along the loop in these loops, and a
+            # last one that the reduction extent cuts in the checked copy below
+            full = f"wir_full_{iv[2:]}"
+            out.append(f"{pad}const int {full} = WIR_EDGE ? min({stop}, {tail}) : {stop};")
         out.append(f"{pad}int {base} = {op.start};")
         # only the aligned body unrolls: the checked body's per-chunk bounds state times m copies
         # spilled (gemm_256_k64: 11 VGPRs, 43 SGPRs), and it runs every trip in the remainder loop
-        out.append(f"{pad}for (; WIR_AL && {base} + {m} <= ({stop}); {base} += {m}) {{")
+        out.append(f"{pad}for (; WIR_AL && {base} + {m} <= ({full}); {base} += {m}) {{")
         for u in range(m):
             self._slot_const[ivn] = (op.start + u) % m
             out.append(f"{pad}  {{")
@@ -1533,9 +1560,38 @@ class CDNA4Lowerer:
             out.append(f"{pad}  }}")
         del self._slot_const[ivn]
         out.append(f"{pad}}}")
-        out.append(f"{pad}for (int {iv} = {base}; {iv} < {stop}; {iv} += 1) {{")
+        out.append(f"{pad}for (int {iv} = {base}; {iv} < {full}; {iv} += 1) {{")
         self._emit_ops(op.body, out, depth + 1)
         out.append(f"{pad}}}")
+        if tail:
+            out.append(f"{pad}for (int {iv} = {full}; WIR_EDGE && {iv} < {stop}; {iv} += 1) {{")
+            out.append(f"{pad}  constexpr bool WIR_AL = false, WIR_INB = false, WIR_EDGE = false;")
+            self._emit_ops(op.body, out, depth + 1)
+            out.append(f"{pad}}}")
+
+    def _checked_tail(self, loop: ForOp) -> Optional[str]:
+        """For a buffer-form loop whose loads all take the loop's own tile:
+        how many tiles lie whole inside every tensor along the loop (C++
+        text).  None where a ring runs behind the loop (its last tiles load
+        in drain steps, which have no checked copy)."""
+        if not self._edge or any(isinstance(o, DrainIndexOp) for o in _walk(self.kernel.body)):
+            return None
+        ivn = loop.induction_var.name
+        counts = []
+        for o in loop.body:
+            if isinstance(o, IntAffineOp):
+                return None
+            if isinstance(o, TMALoadBufOp):
+                sub = o.source.type.sub_tile_type
+                for c, unit, dim in ((o.coords[2], sub.rows, "r"), (o.coords[3], sub.cols, "c")):
+                    if isinstance(c, Value) and c.name == ivn:
+                        counts.append(f"globals.{_cname(o.source.name)[2:]}.{dim} / {unit}")
+        if not counts:
+            return None
+        text = counts[0]
+        for c in counts[1:]:
+            text = f"min({text}, {c})"
+        return text
 
     def _emit_loop_lazy(self, op: ForOp, stop: str, out: List[str], depth: int, fused_at: int) -> None:
         """A loop whose body holds a lazy softmax step (``_match_lazy_softmax``):
@@ -2789,19 +2845,24 @@ class CDNA4Lowerer:
             # with these the aligned body needs no zero-page selects (WIR_INB): every tile it
             # loads lies inside its tensor; a launch that fails them takes the checked body
             checks += "".join(f" && {c}" for c in inb)
+        edge = self._edge_checks(kernel) if inb else []
         src += [
             f"  const bool wir_aligned = {checks};",
             "  auto wir_body = [&](auto wir_tag) {",
             "  constexpr bool WIR_AL = decltype(wir_tag)::value;",
+            *(["  constexpr bool WIR_EDGE = decltype(wir_tag)::edge;  // clamped form of the aligned body"]
+              if self._edge else []),
             f"  constexpr bool WIR_INB = WIR_AL && {'true' if inb else 'false'};  "
             f"// aligned tiles all inside the tensors",
-            "  (void)WIR_INB;",
+            "  (void)WIR_INB;" + (" (void)WIR_EDGE;" if self._edge else ""),
             "  int wir_drain = 0;",
             "  (void)wave_row0; (void)wave_col0; (void)wir_drain;",
             *decls,
         ]
         tail = ["  };",
                 "  if (wir_aligned) wir_body(wir::bool_tag<true>{});",
+                *([f"  else if ({' && '.join(edge)})  // ragged extents: this program's tiles, clamped",
+                   "    wir_body(wir::bool_tag<true, true>{});"] if edge else []),
                 "  else wir_body(wir::bool_tag<false>{});",
                 "}", ""]
         return "\n".join(src + body + tail)
@@ -2909,6 +2970,58 @@ class CDNA4Lowerer:
                     if cond not in conds:
                         conds.append(cond)
         return conds
+
+    def _edge_checks(self, kernel: Kernel) -> List[str]:
+        """Run-time conditions, of one program, under which the WIR_EDGE body
+        loads only from inside its tensors, or ``[]`` when the kernel has no
+        such body.  It is the in-bounds body for extents that are no
+        multiples of the tile: a dimension that a program id indexes needs
+        only the program's tile origin inside (its lanes clamp to the last
+        row or chunk), the loop's last tile may be cut (``_checked_tail``),
+        and the other coordinates are bounded as in ``_in_bounds_checks``.
+        Launches that were in bounds as a whole take the aligned body."""
+        ops = list(_walk(kernel.body))
+        loops = [op for op in kernel.body if isinstance(op, ForOp)]
+        if not self._edge or self._pp_ops or len(loops) != 1:
+            return []
+        loop = loops[0]
+        tail = self._checked_tail(loop) is not None
+        tiles = self._int(loop.stop)
+        if loop.tile_size:
+            tiles = f"(({tiles}) + {loop.tile_size - 1}) / {loop.tile_size}"
+        start = loop.start
+        conds: List[str] = [f"({tiles}) >= {start}"]
+        shifted = {loop.induction_var.name: 0}
+        for o in loop.body:
+            if isinstance(o, IntAffineOp):
+                shifted[o.result.name] = o.add
+        j = 0
+        for op in kernel.body[kernel.body.index(loop) + 1:]:
+            if isinstance(op, MMABufOp):
+                j += 1
+            elif isinstance(op, DrainIndexOp):
+                shifted[op.result.name] = j + op.offset + 1 - start
+        in_loop = {id(o) for o in loop.body}
+        first: Dict[str, int] = {}   # extent -> the largest constant (prologue) tile's end
+        for op in ops:
+            if not isinstance(op, TMALoadBufOp):
+                continue
+            g = f"globals.{_cname(op.source.name)[2:]}"
+            sub = op.source.type.sub_tile_type
+            conds.append(f"wir::Loader<{self.stile(self.resolve(op.buf.name))}, {self.geo.nw}>::clampable({g})")
+            for c, unit, dim in zip(op.coords, (1, 1, sub.rows, sub.cols), "bdrc"):
+                if isinstance(c, int):
+                    first[f"{g}.{dim}"] = max(first.get(f"{g}.{dim}", 0), (c + 1) * unit)
+                elif c.name in _GRID:
+                    conds.append(f"({self._int(c)}) * {unit} < {g}.{dim}")
+                elif c.name in shifted:
+                    # with a checked tail the loop's tiles past the whole ones need no condition
+                    if not (tail and id(op) in in_loop):
+                        conds.append(f"(({tiles}) + {shifted[c.name]}) * {unit} <= {g}.{dim}")
+                else:
+                    return []
+        conds += [f"{v} <= {e}" for e, v in first.items()]
+        return list(dict.fromkeys(conds))
 
     def _wave_tile(self) -> RegTileType:
         """The register tile shape that sets the wavefront slices: the first
@@ -3051,6 +3164,17 @@ class _Sim:
 # ----------------------------------------------------------------------
 # helpers
 # ----------------------------------------------------------------------
+_GRID = ("blockIdx.x", "blockIdx.y", "blockIdx.z")
+
+
+def _buffer_form(kernel: Kernel) -> bool:
+    """Whether the kernel is a ring-buffered product: every tile load goes to a
+    ring slot that a buffered MMA reads."""
+    ops = list(_walk(kernel.body))
+    return (any(isinstance(o, MMABufOp) for o in ops)
+            and not any(isinstance(o, (TMALoadOp, SlotViewOp)) for o in ops))
+
+
 def _walk(ops):
     for op in ops:
         yield op
