@@ -14,8 +14,19 @@ VARIANTS = ["gemm_256_k64", "gemm_128_k64", "gemm_128x64_k64", "gemm_128x32_k64"
             "gemm_128_splitk_k64_b7"]
 
 
+# a ring of five slots: its loop is one copy with run-time slots
+FIVE_SLOTS = "five slots"
+
+
+def _kernel(name):
+    if name != FIVE_SLOTS:
+        return kernels.kernel(name)
+    return kernels._gemm_mi355x(64, block_m=64, block_n=64, wave_m=32, wave_n=32, lds_budget=80 * 1024)
+
+
 def _source(name):
-    src = kernels.lowerer(name).lower(kernels.kernel(name))
+    low = CDNA4Lowerer(CDNA4Target(clamp_edges=True)) if name == FIVE_SLOTS else kernels.lowerer(name)
+    src = low.lower(_kernel(name))
     return src[src.rindex('extern "C" __global__'):]
 
 
@@ -34,14 +45,14 @@ def _eval(expr, ext, pid, n):
     return eval(expr.replace("globals.N", str(n)).replace("/", "//"))   # noqa: S307 - integers only
 
 
-@pytest.mark.parametrize("name", VARIANTS)
+@pytest.mark.parametrize("name", [*VARIANTS, FIVE_SLOTS])
 def test_clamped_body_loads_only_inside_its_tensors(name):
     """Wherever a program's conditions hold, each of its unchecked tile loads
     has its origin inside the tensor in the dimensions that a program id
     indexes (lanes clamp to the last row or chunk there) and lies whole
     inside in the others; the loop's checked copy takes the tiles from
     ``wir_full`` on.  Some swept launches do leave a tensor, and are refused."""
-    kernel, body = kernels.kernel(name), _source(name)
+    kernel, body = _kernel(name), _source(name)
     conds = _conditions(body)
     loop = next(o for o in kernel.body if type(o).__name__ == "ForOp")
     tk, c = loop.tile_size, kernel.outputs[0].type.sub_tile_type
@@ -85,4 +96,5 @@ def test_only_a_loop_without_shifted_rings_has_a_checked_copy():
     """A ring that runs behind the loop loads its last tiles in drain steps,
     which have no checked copy: its reduction extent must be whole tiles."""
     assert "WIR_EDGE && v_i < " in _source("gemm_128_k64")
+    assert "WIR_EDGE && v_i < " in _source(FIVE_SLOTS) and "wir_base_i" not in _source(FIVE_SLOTS)
     assert "WIR_EDGE && v_i < " not in _source("gemm_128_splitk_k64_b7")

@@ -1535,12 +1535,6 @@ class CDNA4Lowerer:
         # one ring size: unroll up to 4 copies; rings of different depths: up to their period 6
         m_max = 4 if m is None or len({f.modulus for o in op.body for f in vars(o).values()
                                         if isinstance(f, BufSlotExpr) and f.value is not None}) == 1 else 6
-        if m is None or m < 2 or m > m_max or not isinstance(op.start, int) or op.step != 1:
-            out.append(f"{pad}for (int {iv} = {self._int(op.start)}; {iv} < {stop}; {iv} += {self._int(op.step)}) {{")
-            self._emit_ops(op.body, out, depth + 1)
-            out.append(f"{pad}}}")
-            return
-        base = f"wir_base_{iv[2:]}"
         tail = self._checked_tail(op)
         full = stop
         if tail:
@@ -1548,19 +1542,23 @@ class CDNA4Lowerer:
             # last one that the reduction extent cuts in the checked copy below
             full = f"wir_full_{iv[2:]}"
             out.append(f"{pad}const int {full} = WIR_EDGE ? min({stop}, {tail}) : {stop};")
-        out.append(f"{pad}int {base} = {op.start};")
-        # only the aligned body unrolls: the checked body's per-chunk bounds state times m copies
-        # spilled (gemm_256_k64: 11 VGPRs, 43 SGPRs), and it runs every trip in the remainder loop
-        out.append(f"{pad}for (; WIR_AL && {base} + {m} <= ({full}); {base} += {m}) {{")
-        for u in range(m):
-            self._slot_const[ivn] = (op.start + u) % m
-            out.append(f"{pad}  {{")
-            out.append(f"{pad}    const int {iv} = {base} + {u};")
-            self._emit_ops(op.body, out, depth + 2)
-            out.append(f"{pad}  }}")
-        del self._slot_const[ivn]
-        out.append(f"{pad}}}")
-        out.append(f"{pad}for (int {iv} = {base}; {iv} < {full}; {iv} += 1) {{")
+        if m is None or m < 2 or m > m_max or not isinstance(op.start, int) or op.step != 1:
+            out.append(f"{pad}for (int {iv} = {self._int(op.start)}; {iv} < {full}; {iv} += {self._int(op.step)}) {{")
+        else:
+            base = f"wir_base_{iv[2:]}"
+            out.append(f"{pad}int {base} = {op.start};")
+            # only the aligned body unrolls: the checked body's per-chunk bounds state times m copies
+            # spilled (gemm_256_k64: 11 VGPRs, 43 SGPRs), and it runs every trip in the remainder loop
+            out.append(f"{pad}for (; WIR_AL && {base} + {m} <= ({full}); {base} += {m}) {{")
+            for u in range(m):
+                self._slot_const[ivn] = (op.start + u) % m
+                out.append(f"{pad}  {{")
+                out.append(f"{pad}    const int {iv} = {base} + {u};")
+                self._emit_ops(op.body, out, depth + 2)
+                out.append(f"{pad}  }}")
+            del self._slot_const[ivn]
+            out.append(f"{pad}}}")
+            out.append(f"{pad}for (int {iv} = {base}; {iv} < {full}; {iv} += 1) {{")
         self._emit_ops(op.body, out, depth + 1)
         out.append(f"{pad}}}")
         if tail:
@@ -1574,7 +1572,8 @@ class CDNA4Lowerer:
         how many tiles lie whole inside every tensor along the loop (C++
         text).  None where a ring runs behind the loop (its last tiles load
         in drain steps, which have no checked copy)."""
-        if not self._edge or any(isinstance(o, DrainIndexOp) for o in _walk(self.kernel.body)):
+        if (not self._edge or not isinstance(loop.start, int) or loop.step != 1
+                or any(isinstance(o, DrainIndexOp) for o in _walk(self.kernel.body))):
             return None
         ivn = loop.induction_var.name
         counts = []
