@@ -7,11 +7,11 @@ import re
 import pytest
 
 from test_lowering import _tile_loads
-from warpir_amd import kernels
+from warpir_amd import api, kernels
 from warpir_amd.lowering import CDNA4Lowerer, CDNA4Target
 
-VARIANTS = ["gemm_256_k64", "gemm_128_k64", "gemm_128x64_k64", "gemm_128x32_k64", "gemm_256x128",
-            "gemm_128_splitk_k64_b7"]
+VARIANTS = ["gemm_256_k64", "gemm_128_k64", "gemm_128_k64_s3", "gemm_128x64_k64", "gemm_64x128_k64",
+            "gemm_64_k64", "gemm_128x32_k64", "gemm_256x128", "gemm_128x256_k64", "gemm_128_splitk_k64_b7"]
 
 
 # a ring of five slots: its loop is one copy with run-time slots
@@ -98,3 +98,18 @@ def test_only_a_loop_without_shifted_rings_has_a_checked_copy():
     assert "WIR_EDGE && v_i < " in _source("gemm_128_k64")
     assert "WIR_EDGE && v_i < " in _source(FIVE_SLOTS) and "wir_base_i" not in _source(FIVE_SLOTS)
     assert "WIR_EDGE && v_i < " not in _source("gemm_128_splitk_k64_b7")
+
+
+@pytest.mark.parametrize("m,n,k,variant", [
+    (256, 256, 256, "gemm_64_k64"), (1, 8, 8, "gemm_64_k64"), (0, 8, 8, None), (8, 8, 0, None),
+    (512, 4096, 8192, "gemm_64x128_k64"), (2048, 2048, 2048, "gemm_128_k64_s3"),
+    (1024, 8192, 8192, None), (4096, 4096, 4096, "gemm_256_k64"), (8192, 8192, 8192, "gemm_256_k64"),
+    (3000, 4104, 4040, "gemm_256_k64"), (128, 8192, 8192, "gemm_128_splitk_k64_b7"),
+    (16384, 16384, 8, None)])
+def test_gemm_route_by_estimated_time(m, n, k, variant):
+    """One tile per CU takes the tile that makes it so; the fallback for
+    strided operands is always a tiled kernel, and every route is built."""
+    got, tiled = api._gemm_route(m, n, k)
+    assert variant in (None, got) and {got, tiled} <= set(kernels.VARIANTS)
+    assert tiled != api.SPLITK_GEMM_VARIANT
+    assert api.gemm_variant(m, n, k) == got

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 # fp32 accumulation, one bf16 rounding of C: at most 2^-8 of the largest value (rel_err's scale)
 TOL = 2.0 ** -8
 
-EDGE_VARIANTS = ["gemm_256_k64", "gemm_256x128", "gemm_128_k64", "gemm_128x64_k64", "gemm_128x32_k64"]
+EDGE_VARIANTS = ["gemm_256_k64", "gemm_256x128", "gemm_128x256_k64", "gemm_128_k64", "gemm_128_k64_s3",
+                 "gemm_128x64_k64", "gemm_64x128_k64", "gemm_64_k64", "gemm_128x32_k64"]
 
 
 def _inside(t, rows, cols, fill):
@@ -55,3 +56,14 @@ def test_ragged_gemm_keeps_infinities_in_their_row_and_column(gpu, variant):
     assert not bool(c[m - 1].isfinite().any()) and not bool(c[:, n - 1].isfinite().any())
     assert bool(c[:m - 1, :n - 1].isfinite().all())
     assert rel_err(c[:m - 1, :n - 1], gemm_ref(a[:m - 1], b[:, :n - 1])) <= TOL
+
+
+@pytest.mark.parametrize("variant", ["gemm_64_k64", "gemm_64x128_k64"])
+@pytest.mark.parametrize("m,n,k", [(64, 128, 64), (128, 128, 256), (192, 256, 320), (1024, 1024, 1024)])
+def test_small_tiles_match_the_256_tile_bit_for_bit(gpu, variant, m, n, k):
+    """Every tiled variant adds the same MFMA products in the same k order."""
+    a, b = seeded_normal((m, k), 4).cuda(), seeded_normal((k, n), 5).cuda()
+    c, ref = (torch.empty(m, n, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    kernels.handle(variant)(A=a, B=b, N=k, C_global=c)
+    kernels.handle("gemm_256_k64")(A=a, B=b, N=k, C_global=ref)
+    assert torch.equal(c, ref)

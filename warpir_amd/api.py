@@ -10,32 +10,88 @@ fallback implementation.
 """
 from __future__ import annotations
 
+import functools
 import math
 from typing import Optional, Tuple
 
 from warpir_amd import kernels
 
 GEMM_VARIANT = "gemm_256_k64"
-SKINNY_GEMM_VARIANT = "gemm_128x32_k64"   # M <= 128: 128x32 tiles, 256 workgroups at N = 8192
-MID_GEMM_VARIANT = "gemm_128_k64"         # fewer 256x256 tiles than CUs: 128x128 tiles
+SKINNY_GEMM_VARIANT = "gemm_64_k64"       # short M, long K, operands that split-K does not take
+MID_GEMM_VARIANT = "gemm_128_k64"         # K unknown, fewer 256x256 tiles than CUs: 128x128 tiles
+
+# Time of one product on the 256 CUs of an MI355X, in microseconds, as a
+# function of its tiles T and 64-deep K steps S:
+#   fixed + S * step + per_mb * (MB of A and B)
+#   step = light + busy * T / 256                                T <= 256
+#        = full * (T // 256), plus the same line from light to
+#          full for the tiles of a last, partial round           T > 256
+# A workgroup's step is slower the more CUs are busy (they share the L2s and
+# the power limit), and `full` is the cost of a step where every CU has
+# another tile to go to.  The constants are least-squares fits (rms 11-13% in
+# log time) to device times of 83 products from 1x312x408 to 14336x12344x1320,
+# ragged and aligned; the variant with the smallest estimate was within 0.6%
+# (geometric mean; 10% at worst) of the fastest one measured.
+#   variant: (tile M, tile N, fixed, light, busy, full, per_mb)
+_TILE_COST = {
+    GEMM_VARIANT: (256, 256, 11.0, 0.837, 0.508, 1.61, 0.0975),
+    "gemm_256x128": (256, 128, 6.62, 0.466, 0.350, 0.950, 0.00306),
+    "gemm_128x256_k64": (128, 256, 7.76, 0.444, 0.168, 0.847, 0.110),
+    "gemm_128_k64_s3": (128, 128, 4.71, 0.293, 0.119, 0.542, 0.0761),
+    "gemm_128x64_k64": (128, 64, 3.41, 0.223, 0.0793, 0.330, 0.0701),
+    "gemm_64x128_k64": (64, 128, 3.68, 0.219, 0.0474, 0.307, 0.103),
+    "gemm_64_k64": (64, 64, 3.26, 0.143, 0.0543, 0.205, 0.0739),
+}
+# split-K (128x128 tiles, `splits` slices) with its reduction:
+#   fixed + S / splits * (light + busy * T * splits / 256) + per_mb * (MB of partials) + per_mb_ab * (MB of A and B)
+_SPLITK_COST = (6.14, 0.459, 0.0407, 0.559, 0.0422)
+
+
+def _tiled_estimate(cost, m: int, n: int, k: int) -> float:
+    bm, bn, fixed, light, busy, full, per_mb = cost
+    rounds, rest = divmod(-(-m // bm) * -(-n // bn), 256)
+    if rounds == 0 or (rounds == 1 and rest == 0):
+        step = light + busy * (rounds + rest / 256)
+    else:
+        step = full * rounds + (light + (full - light) * rest / 256 if rest else 0.0)
+    return fixed + -(-k // 64) * step + per_mb * 2e-6 * k * (m + n)
+
+
+def _splitk_estimate(m: int, n: int, k: int, splits: int) -> float:
+    fixed, light, busy, per_mb, per_mb_ab = _SPLITK_COST
+    programs = -(-m // 128) * -(-n // 128) * splits
+    return (fixed + k / (64 * splits) * (light + busy * programs / 256) + per_mb * 4e-6 * splits * m * n
+            + per_mb_ab * 2e-6 * k * (m + n))
 
 
 def gemm_variant(m: int, n: int, k: Optional[int] = None) -> str:
-    """Kernel variant for an M x N (x K) GEMM on the 256 CUs of one MI355X.
+    """Kernel variant for an M x N (x K) GEMM on the 256 CUs of one MI355X:
+    the tiled variant, or split-K, with the smallest estimated time
+    (``_TILE_COST``).  Measured against the rule it replaced (128x128 tiles
+    below 256 tiles of 256x256, 128x64 for M <= 256), microseconds:
+    512x4096x8192 43.0 vs 72.6, 1024x8192x8192 113.7 vs 146.1,
+    2048x2048x8192 61.9 vs 79.0, 200x4096x4096 14.9 vs 20.4,
+    3000x4104x4040 102 vs 129.  Without K (or with one that is no multiple of
+    8, which no tile load takes) the choice goes by the tile counts alone."""
+    if k is None or k % 8:
+        if m <= 128:
+            return "gemm_128x32_k64"
+        if m <= 256:
+            return "gemm_128x64_k64"
+        if math.ceil(m / 256) * math.ceil(n / 256) < 256:
+            return MID_GEMM_VARIANT
+        return GEMM_VARIANT
+    return _gemm_route(m, n, k)[0]
 
-    Measured at N = K = 8192 with four B operands cycled (512 MiB, so B
-    streams from HBM), microseconds per product: M=64 split-K x4 42.4 vs
-    128x32 67.1; M=128 split-K x4 38.8 vs 128x32 60.4; M=256 128x64 68.5
-    vs split-K x2 69.6."""
-    if m <= 128 and k is not None and splitk_count(m, n, k) >= 4:
-        return SPLITK_GEMM_VARIANT
-    if m <= 128:
-        return SKINNY_GEMM_VARIANT
-    if m <= 256:
-        return "gemm_128x64_k64"
-    if math.ceil(m / 256) * math.ceil(n / 256) < 256:
-        return MID_GEMM_VARIANT
-    return GEMM_VARIANT
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_route(m: int, n: int, k: int) -> Tuple[str, str]:
+    """(variant, variant for operands that split-K does not take)."""
+    tiled, est = min(((v, _tiled_estimate(c, m, n, k)) for v, c in _TILE_COST.items()), key=lambda x: x[1])
+    splits = splitk_count(m, n, k)
+    if splits > 1 and _splitk_estimate(m, n, k, splits) < est:
+        return SPLITK_GEMM_VARIANT, SKINNY_GEMM_VARIANT if m <= 128 else tiled
+    return tiled, tiled
 
 
 # 128x128 tiles, 64-deep K steps; kernel_pass sizes the rings per operand:
@@ -249,9 +305,9 @@ def _splitk_operands_ok(a, b, out) -> bool:
 def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
     """``out[M, N] = a[M, K] @ b[K, N]`` in bf16 with fp32 accumulation.
 
-    The variant follows ``gemm_variant``: 256x256 tiles by default, smaller
-    tiles for outputs with fewer tiles than CUs, split-K for M <= 128 and
-    long K (``workspace`` as in ``gemm_split_k``).  An empty output (M or
+    The variant follows ``gemm_variant``: 256x256 tiles for outputs that fill
+    the chip with them, smaller tiles for others, split-K for few tiles and
+    long K (``workspace`` as in ``gemm_split_k``, taken for M <= 128).  An empty output (M or
     N = 0) launches nothing; K = 0 gives zeros (the kernel's loop runs no
     step and its tile loads read the zero page).
     """
@@ -267,10 +323,17 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
         out = torch.empty(m, n, dtype=torch.bfloat16, device=a.device)
     if variant is None:
         variant = gemm_variant(m, n, k)
+        if workspace is not None:
+            # a workspace is the caller's choice of split-K wherever M <= 128 has at least four
+            # slices, and is not read elsewhere
+            if m <= 128 and splitk_count(m, n, k) >= 4:
+                variant = SPLITK_GEMM_VARIANT
+            else:
+                workspace = None
         if variant == SPLITK_GEMM_VARIANT and not _splitk_operands_ok(a, b, out):
             # the split-K entry points take dense operands only; the tiled
             # kernel reads row-strided views through the globals' row stride
-            variant = SKINNY_GEMM_VARIANT
+            variant = _gemm_route(m, n, k)[1]
     if variant == SPLITK_GEMM_VARIANT:
         return gemm_split_k(a, b, out=out, workspace=workspace)
     kernels.handle(variant)(A=a, B=b, N=k, C_global=out)

@@ -41,6 +41,22 @@ VARIANTS: Dict[str, Callable[[], Kernel]] = {
     # 128x128 block tile (4 wavefronts of 64x64): more workgroups for short M (skinny GEMM).
     "gemm_128_k64": lambda: _gemm_mi355x(64, block_m=128, block_n=128, wave_m=64, wave_n=64,
                                          lds_budget=80 * 1024),
+    # The same tile with a three-slot ring in 96 KiB, one workgroup per CU: loads two steps ahead and
+    # spread over all the step's MFMAs.  The two-slot ring left one step (~600 cycles) for a load to
+    # land: 1024x4096x4096 42.4 -> 34.4 us, 2048x2048x8192 79.0 -> 61.9 us.  (Four slots, eight
+    # waves, or LDS reads two k-steps ahead measured the same; past 256 tiles two workgroups per CU
+    # hide the latency instead and the two-slot ring is 10% faster.)
+    "gemm_128_k64_s3": lambda: _gemm_mi355x(64, block_m=128, block_n=128, wave_m=64, wave_n=64,
+                                            lds_budget=96 * 1024, load_units=12),
+    # 64x64 tiles (four wavefronts of 32x32, two workgroups per CU, four-slot ring) for outputs with
+    # few tiles: 200x4096x4096 14.9 us against 20.4 for 128x64 and 18.0 for 128x32 tiles.
+    "gemm_64_k64": lambda: _gemm_mi355x(64, block_m=64, block_n=64, wave_m=32, wave_n=32,
+                                        lds_budget=64 * 1024, load_units=16),
+    "gemm_64x128_k64": lambda: _gemm_mi355x(64, block_m=64, block_n=128, wave_m=32, wave_n=64,
+                                            lds_budget=80 * 1024, load_units=12),
+    # 128x256 and 256x128 tiles (64x128 / 128x64 per wave, three-slot ring): outputs of about one
+    # such tile per CU, 1024x8192x8192 113.7 us against 146 (128x128) and 167 (256x256)
+    "gemm_128x256_k64": lambda: _gemm_mi355x(64, block_m=128, block_n=256, wave_m=64, wave_n=128),
     # Narrow-N tiles for short M (skinny GEMM): 128 and 256 workgroups at M=128, N=8192,
     # two workgroups per CU (LDS <= 80 KiB).
     "gemm_128x64_k64": lambda: _gemm_mi355x(64, block_m=128, block_n=64, wave_m=64, wave_n=32,
@@ -276,9 +292,13 @@ TARGETS: Dict[str, dict] = {
     "gemm_128_splitk_k32_b14sw": {"dma_spread_whole": True},
 }
 # the products that api.gemm launches run ragged extents in the clamped body
-for _name in ("gemm_256_k64", "gemm_256x128", "gemm_128_k64", "gemm_128x64_k64", "gemm_128x32_k64",
-              "gemm_128_splitk_k64_b7"):
+for _name in ("gemm_256_k64", "gemm_256x128", "gemm_128x256_k64", "gemm_128_k64", "gemm_128_k64_s3",
+              "gemm_128x64_k64", "gemm_64x128_k64", "gemm_64_k64", "gemm_128x32_k64", "gemm_128_splitk_k64_b7"):
     TARGETS[_name] = {**TARGETS.get(_name, {}), "clamp_edges": True}
+# rings of three or more slots: a load has two steps or more to land, so its DMAs spread over all the
+# step's MFMAs (256x128 at 1024x8192x8192: 113.6 us against 119.4 with them in the first half)
+for _name in ("gemm_256x128", "gemm_128x256_k64", "gemm_128_k64_s3", "gemm_64x128_k64", "gemm_64_k64"):
+    TARGETS[_name]["dma_spread_whole"] = True
 # the lazy softmax's row sums on the matrix core (CDNA4Target.rowsum_mfma; config 5 within 0.3-0.7%
 # of the default, the config-4 ping-pong 5% slower)
 for _base in ("mha_d128", "mha_d64_causal"):
