@@ -1890,6 +1890,39 @@ __device__ __forceinline__ int remap_xcd(int hw_id, int total) {
   return (hw_id % NXCD) * per + hw_id / NXCD;
 }
 
+// Program order of causal attention, whose blocks of one head differ in
+// length: hardware id `hw` -> (block x, head y + ny * z), with the longest
+// block of a head at x = nx - 1 (REVERSE) or x = 0.  The first heads run one
+// after another on their XCD, longest block first (remap_xcd: a head's K and V
+// stay in one L2).  The last ones, about TAIL blocks (at least 8 heads), run
+// block length by block length, so the launch ends on the shortest blocks of
+// many heads: with every head in turn the last heads start their longest
+// block late, and the other CUs idle up to that block's time.  Where the tail
+// heads fill the XCDs evenly each XCD takes consecutive heads (query heads
+// that share K and V).
+//
+// TAIL = 2048 is two to four blocks per slot (256 CUs x 2 or 3 workgroups).
+// us, every head in turn / 1024 / 2048 / 4096 / all heads by length:
+//   forward  B1 H32/8 S4096 D128     172 / 139 / 139 / 138 / 142
+//   forward  B16 H16 S4096 D128     1298 / 1209 / 1212 / 1255 / 1385
+//   dK/dV    B16 H16 S1024 D128      266 / 227 / 215 / 216 / 218
+//   forward  B8 H32 S8192 D64       2436 / 2403 / 2370 / 2416 / 3162
+// (all heads by length lose the L2's hold on K and V where they are many and long).
+template <bool REVERSE, int TAIL>
+__device__ __forceinline__ void longest_first(int hw, int nx, int heads, int& x, int& head) {
+  const int tail = min(heads, max(8, TAIL / nx & ~7)), lead = heads - tail;
+  if (hw < lead * nx) {
+    const int id = remap_xcd(hw, lead * nx);
+    x = id % nx;
+    head = id / nx;
+  } else {
+    const int t = hw - lead * nx, u = t % tail;
+    x = t / tail;
+    head = lead + (tail % 8 == 0 ? (u % 8) * (tail / 8) + u / 8 : u);
+  }
+  if (REVERSE) x = nx - 1 - x;
+}
+
 // Grouped tile order over a (tiles_y x tiles_x) grid: GROUP rows of tiles
 // are walked column by column, so consecutive ids reuse B column panels
 // while A row panels stay hot.

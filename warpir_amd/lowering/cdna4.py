@@ -90,6 +90,10 @@ class CDNA4Target:
     mfma: Optional[int] = None
     xcd_remap: bool = True
     group_m: int = 8
+    # Programs of uneven length (causal attention): how many of the last
+    # programs run block length by block length across their heads
+    # (wir::longest_first).  0: every head in turn, longest block first.
+    tail_blocks: int = 2048
     rotate_mma: bool = True
     pingpong: bool = True
     # Modulo variable expansion: unroll ring loops by their slot count so
@@ -2790,6 +2794,8 @@ class CDNA4Lowerer:
                   and op.input.name == "blockIdx.x" and op.mul > 0}
         causal_x = any(isinstance(op, ForOp) and isinstance(op.stop, Value) and self.resolve(op.stop.name) in from_x
                        for op in _walk(kernel.body))
+        causal_start = any(isinstance(op, ForOp) and isinstance(op.start, Value)
+                           and self.resolve(op.start.name) in from_x for op in _walk(kernel.body))
         wpe = max(self.geo.waves_per_eu, 2) if self._ws else self.geo.waves_per_eu
         if wpe > 2 and self.target.waves_per_eu is None:
             # more than two waves per SIMD only where as many workgroups fit in the LDS, and not in
@@ -2813,7 +2819,7 @@ class CDNA4Lowerer:
                     raise LoweringError("persistent_stream takes the non-causal attention forward")
                 body = ["  if constexpr (WIR_AL) {", *self._stream_lines, "  } else {", *body, "  }"]
         else:
-            pid = _pid_code(dims, self.target, reverse_x=causal_x)
+            pid = _pid_code(dims, self.target, reverse_x=causal_x, uneven=causal_x or causal_start)
         src = [
             *([f"{HIPCC_FLAGS_MARKER} -mllvm -amdgpu-mfma-vgpr-form=1"] if self.target.mfma_vgpr_form else []),
             "// Generated by warpir_amd.lowering.CDNA4Lowerer for gfx950 -- do not edit.",
@@ -3238,11 +3244,23 @@ def _flt(x: float) -> str:
     return repr(float(x)) + "f"
 
 
-def _pid_code(dims: int, target: CDNA4Target, reverse_x: bool) -> List[str]:
+def _pid_code(dims: int, target: CDNA4Target, reverse_x: bool, uneven: bool = False) -> List[str]:
+    """Program ids from the hardware ids.  ``uneven``: the programs of one
+    head differ in length along x (causal loops; the longest at x = nx - 1
+    with ``reverse_x``, else at 0), and about the last ``tail_blocks`` of them
+    run block length by block length (``wir::longest_first``)."""
     lines = [
         "  const int nx_ = gridDim.x, ny_ = gridDim.y, nz_ = gridDim.z;",
         "  const int hw_ = blockIdx.x + nx_ * (blockIdx.y + ny_ * blockIdx.z);",
     ]
+    if uneven and dims == 3 and target.xcd_remap and target.tail_blocks:
+        return lines + [
+            "  int pid_x, head_;",
+            f"  wir::longest_first<{'true' if reverse_x else 'false'}, {target.tail_blocks}>"
+            "(hw_, nx_, ny_ * nz_, pid_x, head_);",
+            "  const int pid_y = head_ % ny_, pid_z = head_ / ny_;",
+            "  (void)pid_x; (void)pid_y; (void)pid_z;",
+        ]
     if target.xcd_remap:
         lines.append("  const int lid_ = wir::remap_xcd(hw_, nx_ * ny_ * nz_);")
     else:
