@@ -15,6 +15,15 @@ import math
 from typing import Optional, Tuple
 
 from warpir_amd import kernels
+from warpir_amd.plans import Plans, Recording
+
+# Plans of the calls below, by flags: gemm 0; attention_forward and
+# attention_backward the causal bit.  A stream of calls, before -> after: gemm
+# 256^3 10.7 -> 4.4 us and attention_forward B1 H8 S512 D64 16.0 -> 10.1 us, now
+# the kernels' own time and the gap between launches.
+_gemm_plans = Plans("gemm")
+_forward_plans = Plans("attention_forward")
+_backward_plans = Plans("attention_backward")
 
 GEMM_VARIANT = "gemm_256_k64"
 SKINNY_GEMM_VARIANT = "gemm_64_k64"       # short M, long K, operands that split-K does not take
@@ -313,14 +322,20 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
     """
     import torch
 
+    planned = variant is None and workspace is None
+    if planned:
+        done = _gemm_plans.run(0, a, b, out)
+        if done is not None:
+            return done
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[0]:
         raise ValueError(f"gemm: shapes {tuple(a.shape)} @ {tuple(b.shape)} do not chain")
     m, k = a.shape
     n = b.shape[1]
     if k % 8 or n % 8:
         raise ValueError("gemm: K and N must be multiples of 8 (16-byte rows)")
+    rec = Recording(a, b, out)
     if out is None:
-        out = torch.empty(m, n, dtype=torch.bfloat16, device=a.device)
+        out = rec.alloc(torch.empty(m, n, dtype=torch.bfloat16, device=a.device))
     if variant is None:
         variant = gemm_variant(m, n, k)
         if workspace is not None:
@@ -335,9 +350,39 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
             # kernel reads row-strided views through the globals' row stride
             variant = _gemm_route(m, n, k)[1]
     if variant == SPLITK_GEMM_VARIANT:
-        return gemm_split_k(a, b, out=out, workspace=workspace)
-    kernels.handle(variant)(A=a, B=b, N=k, C_global=out)
+        splits = splitk_count(m, n, k)
+        if planned and a.is_cuda:
+            workspace = rec.alloc(torch.empty(splits * m * n, dtype=torch.float32, device=a.device))
+        gemm_split_k(a, b, out=out, workspace=workspace)
+        if planned and a.is_cuda:
+            _record_split_k(rec, a, b, out, workspace, splits)
+            _gemm_plans.add(0, rec, out)
+        return out
+    handle = kernels.handle(variant)
+    handle(A=a, B=b, N=k, C_global=out)
+    if planned and m and n and k and a.is_cuda:
+        rec.kernel(handle, A=a, B=b, N=k, C_global=out)
+        _gemm_plans.add(0, rec, out)
     return out
+
+
+def _record_split_k(rec: Recording, a, b, out, ws, splits: int) -> None:
+    """The two launches of ``wir_gemm_splitk``: the slices of A and B along
+    the depth of their globals, then the reduction."""
+    import ctypes
+
+    class Reduce(ctypes.Structure):
+        _fields_ = [("partials", ctypes.c_void_p), ("out", ctypes.c_void_p), ("n", ctypes.c_longlong),
+                    ("split_stride", ctypes.c_longlong), ("splits", ctypes.c_int)]
+
+    (m, k), n = a.shape, b.shape[1]
+    kc = k // splits
+    a4, b4, ws4 = a.view(1, m, splits, kc).transpose(1, 2), b.view(1, splits, kc, n), ws.view(1, splits, m, n)
+    rec.kernel(kernels.handle(SPLITK_GEMM_VARIANT), A=a4, B=b4, N=kc, C_global=ws4,
+               addend={"A": (a, 0), "B": (b, 0), "C_global": (ws, 0)})
+    _, reduce_fn = _splitk_functions(SPLITK_GEMM_VARIANT)
+    rec.raw(reduce_fn, ((m * n // 8 + 255) // 256, 1, 1), (256, 1, 1), Reduce(0, 0, m * n, m * n, splits),
+            [(Reduce.partials.offset, rec.slot(ws), 0), (Reduce.out.offset, rec.slot(out), 0)])
 
 
 def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
@@ -348,6 +393,11 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     """
     import torch
 
+    planned = variant is None
+    if planned:
+        done = _forward_plans.run(1 if causal else 0, q, k, v, out, lse)
+        if done is not None:
+            return done
     bsz, heads, seq, d = q.shape
     hr = _head_ratio("attention_forward", q, k, v)
     if variant is None:
@@ -361,16 +411,20 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     kv_tile = next(o for o in _loops(handle.kernel)).tile_size
     if seq % kv_tile:
         raise ValueError(f"attention_forward: S={seq} must be a multiple of the KV tile {kv_tile}")
+    rec = Recording(q, k, v, out, lse)
     if out is None:
-        out = torch.empty_like(q)
+        out = rec.alloc(torch.empty_like(q))
     if lse is None:
-        lse = torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device)
+        lse = rec.alloc(torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device))
+    args = dict(Q=q, K=k, V=v, N=seq, O=out, L=lse)
     if any(v_.name == "HR" for v_ in handle.kernel.inputs):
-        handle(Q=q, K=k, V=v, N=seq, HR=hr, O=out, L=lse)
+        args["HR"] = hr
     elif hr > 1:
         raise ValueError(f"attention_forward: variant {variant} takes no grouped-query heads")
-    else:
-        handle(Q=q, K=k, V=v, N=seq, O=out, L=lse)
+    handle(**args)
+    if planned and q.is_cuda and out.numel() and k.numel():
+        rec.kernel(handle, **args)
+        _forward_plans.add(1 if causal else 0, rec, out, lse)
     return out, lse
 
 
@@ -401,6 +455,11 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     same gradients with dQ by atomic adds)."""
     import torch
 
+    planned = workspace is None
+    if planned:
+        done = _backward_plans.run(1 if causal else 0, q, k, v, o, lse, do, dq, dk, dv, dvec)
+        if done is not None:
+            return done
     if q.dim() != 4 or not (q.shape == o.shape == do.shape):
         raise ValueError("attention_backward: q, o, do must share one [B, H, S, D] shape")
     hr = _head_ratio("attention_backward", q, k, v)
@@ -409,36 +468,52 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
         raise ValueError(f"attention_backward: D must be 64 or 128 and S a multiple of 64 (got D={d}, S={seq})")
     if tuple(lse.shape) != (bsz, heads, seq) or lse.dtype != torch.float32:
         raise ValueError("attention_backward: lse must be fp32 [B, H, S]")
-    dq = torch.empty_like(q) if dq is None else dq
-    dk = torch.empty_like(k) if dk is None else dk
-    dv = torch.empty_like(v) if dv is None else dv
-    dvec = torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device) if dvec is None else dvec
-    lse2 = torch.empty_like(lse)   # the LSE in log2 units, for the dK/dV kernel
-    kernels.handle(f"mha_bwd_prep_d{d}")(O=o, dO=do, L=lse, Dv=dvec, L2=lse2)
-    sfx = "_causal" if causal else ""
+    rec = Recording(q, k, v, o, lse, do, dq, dk, dv, dvec)
+    dq = rec.alloc(torch.empty_like(q)) if dq is None else dq
+    dk = rec.alloc(torch.empty_like(k)) if dk is None else dk
+    dv = rec.alloc(torch.empty_like(v)) if dv is None else dv
+    dvec = rec.alloc(torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device)) if dvec is None else dvec
+    lse2 = rec.alloc(torch.empty_like(lse))   # the LSE in log2 units, for the dK/dV kernel
+    # (handle, arguments, views) of each launch in order
+    launches = [(kernels.handle(f"mha_bwd_prep_d{d}"), dict(O=o, dO=do, L=lse, Dv=dvec, L2=lse2), None)]
+    sfx = ("_causal" if causal else "") + ("_gqa" if hr > 1 else "")
+    dq_args = dict(Q=q, K=k, V=v, dO=do, L=lse, Dv=dvec, N=seq, dQ=dq)
+    dkdv_args = dict(Q=q, K=k, V=v, dO=do, L2=lse2, Dv=dvec, N=seq)
+    views = None
     if hr == 1:
-        kernels.handle(f"mha_bwd_dq_d{d}{sfx}")(Q=q, K=k, V=v, dO=do, L=lse, Dv=dvec, N=seq, dQ=dq)
-        kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}")(Q=q, K=k, V=v, dO=do, L2=lse2, Dv=dvec, N=seq, dK=dk, dV=dv)
-        return dq, dk, dv
-    numel = q.numel()
-    if workspace is None:
-        workspace = torch.empty(2 * numel, dtype=torch.float32, device=q.device)
-    if workspace.dtype != torch.float32 or workspace.numel() < 2 * numel or not workspace.is_contiguous():
-        raise ValueError(f"attention_backward: workspace must be contiguous fp32 with >= {2 * numel} elements")
-    dk_part = workspace[:numel].view(q.shape)
-    dv_part = workspace[numel:2 * numel].view(q.shape)
-    kernels.handle(f"mha_bwd_dq_d{d}{sfx}_gqa")(Q=q, K=k, V=v, dO=do, L=lse, Dv=dvec, N=seq, HR=hr, dQ=dq)
-    kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}_gqa")(Q=q, K=k, V=v, dO=do, L2=lse2, Dv=dvec, N=seq, HR=hr,
-                                                  dK_part=dk_part, dV_part=dv_part)
-    _group_reduce(dk_part, dk, hr)
-    _group_reduce(dv_part, dv, hr)
+        dkdv_args.update(dK=dk, dV=dv)
+    else:
+        numel = q.numel()
+        if workspace is None:
+            workspace = rec.alloc(torch.empty(2 * numel, dtype=torch.float32, device=q.device))
+        if workspace.dtype != torch.float32 or workspace.numel() < 2 * numel or not workspace.is_contiguous():
+            raise ValueError(f"attention_backward: workspace must be contiguous fp32 with >= {2 * numel} elements")
+        dk_part = workspace[:numel].view(q.shape)
+        dv_part = workspace[numel:2 * numel].view(q.shape)
+        views = {"dK_part": (workspace, 0), "dV_part": (workspace, 4 * numel)}
+        dq_args["HR"] = hr
+        dkdv_args.update(HR=hr, dK_part=dk_part, dV_part=dv_part)
+    launches += [(kernels.handle(f"mha_bwd_dq_d{d}{sfx}"), dq_args, None),
+                 (kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}"), dkdv_args, views)]
+    for handle, args, _ in launches:
+        handle(**args)
+    reductions = []
+    if hr > 1:
+        reductions = [(_group_reduce(dk_part, dk, hr), 0, dk), (_group_reduce(dv_part, dv, hr), 4 * numel, dv)]
+    if planned and q.is_cuda and q.numel() and k.numel():
+        for handle, args, seen in launches:
+            rec.kernel(handle, addend=seen, **args)
+        for (grid, args), off, grad in reductions:
+            rec.raw(_group_reduce_kernel._function, grid, (256, 1, 1), args,
+                    [(type(args).partials.offset, rec.slot(workspace), off), (type(args).out.offset, rec.slot(grad), 0)])
+        _backward_plans.add(1 if causal else 0, rec, dq, dk, dv)
     return dq, dk, dv
 
 
 _group_reduce_kernel = None
 
 
-def _group_reduce(partials, out, splits: int) -> None:
+def _group_reduce(partials, out, splits: int):
     """``out[g] = bf16(sum_r partials[g * splits + r])`` over the key/value head
     groups of a ``[B, H, S, D]`` fp32 contribution tensor (``splitk_reduce.hip``)."""
     import ctypes
@@ -456,13 +531,15 @@ def _group_reduce(partials, out, splits: int) -> None:
     if not out.is_contiguous() or out.dtype.itemsize != 2:
         raise ValueError("attention_backward: dk / dv must be contiguous bf16")
     if out.numel() == 0:
-        return
+        return None
     n = out.shape[-2] * out.shape[-1]
     groups = out.numel() // n
     if n % 8 or partials.numel() != groups * splits * n:
         raise ValueError("attention_backward: grouped reduction needs S * D % 8 == 0 and matching shapes")
     args = Args(partials.data_ptr(), out.data_ptr(), n, groups, splits)
-    _group_reduce_kernel.launch(((groups * n // 8 + 255) // 256, 1, 1), (256, 1, 1), args)
+    grid = ((groups * n // 8 + 255) // 256, 1, 1)
+    _group_reduce_kernel.launch(grid, (256, 1, 1), args)
+    return grid, args
 
 
 def attention_backward_flops(bsz: int, heads: int, seq: int, d: int, causal: bool = False) -> float:
