@@ -407,6 +407,10 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
             raise ValueError(f"attention_forward: no kernel variant for D={d}, causal={causal}")
         if hr > 1:
             variant += "_gqa"
+        elif variant == "mha_d128" and -(-seq // 256) * heads * bsz < 256:
+            # 256-row blocks leave CUs idle: 128-row blocks of the same softmax
+            # (B1 H16 S2048 49.9 -> 43.4 us, B1 H8 S512 16.7 -> 13.6 us)
+            variant = "mha_d128_w4"
     handle = kernels.handle(variant)
     kv_tile = next(o for o in _loops(handle.kernel)).tile_size
     if seq % kv_tile:
@@ -417,6 +421,9 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     if lse is None:
         lse = rec.alloc(torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device))
     args = dict(Q=q, K=k, V=v, N=seq, O=out, L=lse)
+    if planned and _split_kv_fits(bsz, heads, seq, causal, k, v):
+        _attention_split_kv(handle, args, hr, causal, rec)
+        return out, lse
     if any(v_.name == "HR" for v_ in handle.kernel.inputs):
         args["HR"] = hr
     elif hr > 1:
@@ -426,6 +433,50 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
         rec.kernel(handle, **args)
         _forward_plans.add(1 if causal else 0, rec, out, lse)
     return out, lse
+
+
+def _split_kv_fits(bsz: int, heads: int, seq: int, causal: bool, k, v) -> bool:
+    """Whether the forward goes to the split-key kernel
+    (``attn_splitkv.hip``, 32 query rows per program, one program per CU).
+    It wins while its programs fit the CUs once, and causal ones, half of them
+    short, twice.  us, tiled -> split: B1 H8 S512 D64 10.3 -> 6.0 (128
+    programs), S1024 16.8 -> 9.2 (256), S1024 D128 26.6 -> 15.9; at 512
+    programs S2048 D64 30.0 -> 26.5 and D128 46.5 -> 48.5, causal 29.3 -> 18.5
+    and 41.1 -> 31.1; at 1024 B2 H8 S2048 D64 31.8 -> 49.9.  Its lane offsets
+    are 32-bit."""
+    return (0 < bsz * heads * (seq // 32) <= (512 if causal else 256)
+            and all(0 <= t.stride(2) < 1 << 23 for t in (k, v)))
+
+
+_split_kv_kernels: dict = {}
+
+
+def _attention_split_kv(handle, args: dict, hr: int, causal: bool, rec: Recording) -> None:
+    """Launch the split-key forward on the arguments of the tiled kernel
+    *handle*, which validates and packs them, and keep the call's plan."""
+    import ctypes
+
+    import torch
+
+    from warpir_amd.runtime import GL, RawKernel
+
+    class Args(ctypes.Structure):
+        _fields_ = [("Q", GL), ("K", GL), ("V", GL), ("N", ctypes.c_int), ("HR", ctypes.c_int), ("O", GL), ("L", GL)]
+
+    if "HR" in handle.args_type.__dict__:
+        args = {**args, "HR": hr}
+    packed, _cfg, device, _empty = handle.pack(args)
+    name = f"wir_attn_splitkv_d{args['Q'].shape[3]}" + ("_causal" if causal else "")
+    kernel = _split_kv_kernels.get(name)
+    if kernel is None:
+        kernel = _split_kv_kernels.setdefault(name, RawKernel("attn_splitkv.hsaco", name))
+    packed = Args(packed.Q, packed.K, packed.V, args["N"], hr, packed.O, packed.L)
+    bsz, heads, seq, _ = args["Q"].shape
+    grid, block = (seq // 32, heads, bsz), (256, 1, 1)
+    kernel.launch(grid, block, packed, stream=torch.cuda.current_stream(device).cuda_stream)
+    rec.raw(kernel._function, grid, block, packed,
+            [(getattr(Args, f).offset, rec.slot(args[f]), 0) for f in "QKVOL"])
+    _forward_plans.add(1 if causal else 0, rec, args["O"], args["L"])
 
 
 def _head_ratio(fn: str, q, k, v) -> int:
