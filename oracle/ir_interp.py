@@ -43,7 +43,7 @@ import torch
 from warpir_amd.ir import (
     AddOp, AllocSharedOp, BufSlotExpr, CausalMaskOp, ColVecType, CopyOp, DivRowOp, DrainIndexOp, Exp2Op,
     ForOp, GPUType, IntAffineOp, IntDivOp, Kernel, LoadVecOp, Log2Op, MMABufOp, MMAOp, MulOp, MulRowOp, MulScalarOp,
-    NegInftyOp, PipelineStageOp, ReduceSlicesOp, RegTileType, RowMaxOp, RowSumOp, RowVecType, SlotViewOp, SubColOp, SubOp, SubRowOp, LazyMaxOp,
+    NegInftyOp, PipelineStageOp, ReduceSlicesOp, RegTileType, RowDotOp, RowMaxOp, RowSumOp, RowVecType, SlotViewOp, SubColOp, SubOp, SubRowOp, LazyMaxOp,
     TMALoadBufOp, TMALoadOp, TMAStoreOp, Value, WaitBufOp, WaitOp, YieldOp, ZeroOp,
 )
 
@@ -257,6 +257,8 @@ class Interpreter:
         elif isinstance(op, LazyMaxOp):
             prev, cand = g(op.prev), g(op.cand)
             s(op.result, torch.where(cand > prev + op.slack, cand, prev))
+        elif isinstance(op, RowDotOp):
+            s(op.result, (g(op.a).float() * g(op.b).float()).sum(dim=1))
         elif isinstance(op, LoadVecOp) and not op.coords:
             s(op.result, g(op.source)[:, 0].clone())   # from an fp32 L x 1 shared tile
         elif isinstance(op, LoadVecOp):

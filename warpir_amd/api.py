@@ -498,10 +498,11 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     each query head's fp32 dK / dV contribution into ``workspace`` (fp32, at
     least ``2 * B * H * S * D`` elements, allocated if omitted) and a HIP
     reduction sums the ``H / H_kv`` contributions of every key/value head
-    into bf16 ``dK`` / ``dV``.  Three WarpIR kernels run
-    on the current stream: ``Dv = rowsum(dO * O)`` (into ``dvec``, fp32
-    ``[B, H, S]``, allocated if omitted) together with the LSE in log2 units,
-    the query-major dQ kernel and the key-major dK/dV kernel (the reference's TK backward,
+    into bf16 ``dK`` / ``dV``.  Two WarpIR kernels run
+    on the current stream: the query-major dQ kernel, which also writes
+    ``Dv = rowsum(dO * O)`` (into ``dvec``, fp32 ``[B, H, S]``, allocated if
+    omitted) and the LSE in log2 units, and the key-major dK/dV kernel, which
+    reads them (the reference's TK backward,
     ``kernel_examples/attention/mha_h100.cu:253-303,482-642``, computes the
     same gradients with dQ by atomic adds)."""
     import torch
@@ -525,10 +526,8 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     dv = rec.alloc(torch.empty_like(v)) if dv is None else dv
     dvec = rec.alloc(torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device)) if dvec is None else dvec
     lse2 = rec.alloc(torch.empty_like(lse))   # the LSE in log2 units, for the dK/dV kernel
-    # (handle, arguments, views) of each launch in order
-    launches = [(kernels.handle(f"mha_bwd_prep_d{d}"), dict(O=o, dO=do, L=lse, Dv=dvec, L2=lse2), None)]
     sfx = ("_causal" if causal else "") + ("_gqa" if hr > 1 else "")
-    dq_args = dict(Q=q, K=k, V=v, dO=do, L=lse, Dv=dvec, N=seq, dQ=dq)
+    dq_args = dict(Q=q, K=k, V=v, dO=do, O=o, L=lse, N=seq, dQ=dq, Dv=dvec, L2=lse2)
     dkdv_args = dict(Q=q, K=k, V=v, dO=do, L2=lse2, Dv=dvec, N=seq)
     views = None
     if hr == 1:
@@ -544,8 +543,9 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
         views = {"dK_part": (workspace, 0), "dV_part": (workspace, 4 * numel)}
         dq_args["HR"] = hr
         dkdv_args.update(HR=hr, dK_part=dk_part, dV_part=dv_part)
-    launches += [(kernels.handle(f"mha_bwd_dq_d{d}{sfx}"), dq_args, None),
-                 (kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}"), dkdv_args, views)]
+    # (handle, arguments, views) of each launch in order
+    launches = [(kernels.handle(f"mha_bwd_dq_prep_d{d}{sfx}"), dq_args, None),
+                (kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}"), dkdv_args, views)]
     for handle, args, _ in launches:
         handle(**args)
     reductions = []

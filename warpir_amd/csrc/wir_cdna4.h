@@ -1236,6 +1236,24 @@ __device__ __forceinline__ float lane_group_reduce(float x, F op) {
 struct OpMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
 struct OpAdd { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
 
+// out[r] = sum over columns of a[r, c] * b[r, c], both held as row fragments
+// (lane = row, the columns split over the lane groups): fp32, exact products.
+template <int MS, int R, int RB, int KS>
+__device__ __forceinline__ void row_dot(RVec<MS, R>& out, const RowFrags<MS, RB, KS>& a,
+                                        const RowFrags<MS, RB, KS>& b) {
+  static_assert(RB == RVec<MS, R>::RB, "one value per row block");
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        part[j & 3] = __builtin_fmaf((float)a.f[rb][ks][j], (float)b.f[rb][ks][j], part[j & 3]);
+    out.v[rb] = lane_group_reduce<MS>((part[0] + part[1]) + (part[2] + part[3]), OpAdd());
+  }
+}
+
 // out[r] = op(op_c tile[r, c], prev[r]).
 template <int MS, int R, int C, class F>
 __device__ __forceinline__ void row_reduce(RVec<MS, R>& out, const RTile<MS, R, C>& t, const RVec<MS, R>& prev,

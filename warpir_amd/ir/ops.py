@@ -274,6 +274,17 @@ class SubColOp(Op):
 
 
 @dataclass(frozen=True)
+class RowDotOp(Op):
+    """*Additive.* ``result[r] = sum_c a[r, c] * b[r, c]`` in fp32, a col_vec of
+    two shared bf16 tiles of one shape (``Dv = rowsum(dO * O)`` of the
+    attention backward, in the kernel that holds dO)."""
+
+    result: Value
+    a: Value
+    b: Value
+
+
+@dataclass(frozen=True)
 class LazyMaxOp(Op):
     """*Additive.* ``result = cand if cand > prev + slack else prev`` element-wise.
 

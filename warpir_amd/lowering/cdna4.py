@@ -47,7 +47,7 @@ from typing import Dict, List, Optional, Sequence, Tuple, Union
 from warpir_amd.ir.ops import (
     AddOp, AllocSharedOp, BufSlotExpr, CausalMaskOp, CopyOp, DivRowOp, DrainIndexOp, Exp2Op, ForOp,
     IntAffineOp, IntDivOp, Kernel, LoadVecOp, Log2Op, MMABufOp, MMAOp, MulOp, MulRowOp, MulScalarOp, NegInftyOp,
-    LazyMaxOp, Op, PipelineStageOp, ReduceSlicesOp, RowMaxOp, RowSumOp, SubColOp, SubOp, SubRowOp, TMALoadBufOp, TMALoadOp, TMAStoreOp, Value,
+    LazyMaxOp, Op, PipelineStageOp, ReduceSlicesOp, RowDotOp, RowMaxOp, RowSumOp, SubColOp, SubOp, SubRowOp, TMALoadBufOp, TMALoadOp, TMAStoreOp, Value,
     WaitBufOp, WaitOp, YieldOp, ZeroOp,
 )
 from warpir_amd.ir.ops import SlotViewOp
@@ -1246,6 +1246,12 @@ class CDNA4Lowerer:
         if isinstance(op, SubColOp):
             w(f"{pad}wir::col_apply({self._var(op.result)}, {self._var(op.tile)}, {self._var(op.vec)}, "
               f"[](float x, float s) {{ return x - s; }});")
+            return
+        if isinstance(op, RowDotOp):
+            frags = [self._register_tiles.get(self.resolve(v.name)) for v in (op.a, op.b)]
+            if None in frags:
+                raise LoweringError("row_dot reads two tiles held as row fragments in registers")
+            w(f"{pad}wir::row_dot({self._var(op.result)}, {frags[0][0]}, {frags[1][0]});")
             return
         if isinstance(op, LoadVecOp) and isinstance(op.source.type, SharedTileType):
             ptr, _key = self._tile_ptr(op.source)
@@ -2729,10 +2735,18 @@ class CDNA4Lowerer:
                     for x in _values_in(v):
                         if self.resolve(x.name) != name:
                             continue
-                        if not (isinstance(o, MMAOp) and o.transpose_b and f == "a"):
+                        if not (isinstance(o, MMAOp) and o.transpose_b and f == "a" or isinstance(o, RowDotOp)):
                             uses_ok = False
             if uses_ok:
                 out[name] = info
+        # the other operand of a row_dot, read by nothing else, takes the same fragments
+        for dot in [o for o in self.kernel.body if isinstance(o, RowDotOp)]:
+            for mine, other in ((dot.a, dot.b), (dot.b, dot.a)):
+                name, info = self.resolve(mine.name), out.get(self.resolve(other.name))
+                uses = [o for o in _walk(self.kernel.body) if not isinstance(o, WaitOp)
+                        and any(self.resolve(x.name) == name for f in vars(o).values() for x in _values_in(f))]
+                if info and name not in out and len(uses) == 2 and isinstance(uses[0], TMALoadOp) and uses[1] is dot:
+                    out[name] = (f"hf_{_cname(name)[2:]}", info[1], info[2], None)
         return out
 
     def _hoistable(self) -> Dict[str, tuple]:

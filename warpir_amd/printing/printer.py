@@ -37,6 +37,7 @@ from warpir_amd.ir.ops import (
     RowSumOp,
     SlotViewOp,
     SubOp,
+    RowDotOp,
     SubColOp,
     LazyMaxOp,
     SubRowOp,
@@ -132,6 +133,7 @@ _LINE: Dict[type, Callable[[Op], str]] = {
     IntAffineOp: lambda op: (
         f"{op.result!r} = int_affine({_coord(op.input)}, {op.mul}, {op.add})"
     ),
+    RowDotOp: lambda op: _call(op, "row_dot", op.a, op.b),
     SubColOp: lambda op: _call(op, "sub_col", op.tile, op.vec),
     LoadVecOp: lambda op: f"{op.result!r} = load_vec({op.source!r}, {_coords(op.coords)})",
     LazyMaxOp: lambda op: f"{op.result!r} = lazy_max({op.prev!r}, {op.cand!r}, {op.slack})",

@@ -40,6 +40,7 @@ from warpir_amd.ir import (
     NegInftyOp,
     RegTileType,
     ReduceSlicesOp,
+    RowDotOp,
     RowMaxOp,
     RowSumOp,
     RowVecType,
@@ -363,17 +364,25 @@ def build_mha_bwd_prep_kernel(d: int = 128, block_q: int = 128, wave_rows: int =
 
 
 def build_mha_bwd_dq_kernel(d: int = 128, block_q: int = 128, block_kv: int = 64, wave_rows: int = 32,
-                            name: str = "mha_bwd_dq", causal: bool = False, gqa: bool = False) -> Kernel:
+                            name: str = "mha_bwd_dq", causal: bool = False, gqa: bool = False,
+                            prep: bool = False) -> Kernel:
     """``dQ`` of attention forward, query-major: one program per query tile
     ``(blockIdx.x, head, batch)``; the loop walks key tiles.  With
     ``causal`` it stops at the query tile's last row and masks the scores
     as the causal forward does; with ``gqa`` K and V come from key/value
-    head ``head // HR`` (an extra int input)."""
+    head ``head // HR`` (an extra int input).
+
+    ``prep`` (additive): the program also does the work of
+    ``build_mha_bwd_prep_kernel`` for its rows -- it holds dO anyway, so
+    ``Dv = rowsum(dO * O)`` costs one read of O -- and ``Dv`` and ``L2`` are
+    outputs after ``dQ`` instead of ``Dv`` being an input (``O`` takes its
+    place, ahead of ``L``)."""
     scale = 1.0 / math.sqrt(d)
     q_glob, vec_glob, q_tile = _bwd_globals(d, block_q)
     kv_glob, _, kv_tile = _bwd_globals(d, block_kv)
     Q, K, V, dO = Value("Q", q_glob), Value("K", kv_glob), Value("V", kv_glob), Value("dO", q_glob)
     L, Dv, dQ = Value("L", vec_glob), Value("Dv", vec_glob), Value("dQ", q_glob)
+    O, L2, o_sh = Value("O", q_glob), Value("L2", vec_glob), Value("o_shared", q_tile)
     n_kv = Value("N", IntType())
     q_idx, head, batch = (Value(n, IntType()) for n in ("blockIdx.x", "blockIdx.y", "blockIdx.z"))
     bh = (batch, head)
@@ -430,16 +439,22 @@ def build_mha_bwd_dq_kernel(d: int = 128, block_q: int = 128, block_kv: int = 64
         *head_map,
         TMALoadOp(result=q_sh, source=Q, coords=(*bh, q_idx, 0)),
         TMALoadOp(result=do_sh, source=dO, coords=(*bh, q_idx, 0)),
-        WaitOp(values=(q_sh, do_sh)),
+        *([TMALoadOp(result=o_sh, source=O, coords=(*bh, q_idx, 0))] if prep else []),
+        WaitOp(values=(q_sh, do_sh, o_sh) if prep else (q_sh, do_sh)),
         LoadVecOp(result=lse, source=L, coords=(*bh, q_idx, 0)),
-        LoadVecOp(result=dvec, source=Dv, coords=(*bh, q_idx, 0)),
+        RowDotOp(result=dvec, a=do_sh, b=o_sh) if prep
+        else LoadVecOp(result=dvec, source=Dv, coords=(*bh, q_idx, 0)),
         MulScalarOp(result=lse2, input=lse, scalar=LOG2E),
+        *([TMAStoreOp(source=dvec, dest=Dv, coords=(*bh, q_idx, 0)),
+           TMAStoreOp(source=lse2, dest=L2, coords=(*bh, q_idx, 0))] if prep else []),
         ZeroOp(result=dq_init),
         *prologue,
         loop,
         MulScalarOp(result=dq_out, input=dq_final, scalar=scale),
         TMAStoreOp(source=dq_out, dest=dQ, coords=(*bh, q_idx, 0)),
     )
+    if prep:
+        return Kernel(name=name, inputs=(Q, K, V, dO, O, L, n_kv, *extra_inputs), outputs=(dQ, Dv, L2), body=body)
     return Kernel(name=name, inputs=(Q, K, V, dO, L, Dv, n_kv, *extra_inputs), outputs=(dQ,), body=body)
 
 
