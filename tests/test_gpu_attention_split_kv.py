@@ -92,3 +92,7 @@ def test_few_256_row_blocks_take_128_row_blocks(gpu, taken):
     o, lse = api.attention_forward(q, k, v)
     o2, lse2 = api.attention_forward(q, k, v, variant="mha_d128_w4")
     assert not taken and torch.equal(o, o2) and torch.equal(lse, lse2)
+    q, k, v = (seeded_normal((6, 8, 896, 128), s).cuda() for s in range(3))   # 336 of them: 256-row blocks
+    o, lse = api.attention_forward(q, k, v)
+    o2, lse2 = api.attention_forward(q, k, v, variant="mha_d128")
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)

@@ -407,9 +407,10 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
             raise ValueError(f"attention_forward: no kernel variant for D={d}, causal={causal}")
         if hr > 1:
             variant += "_gqa"
-        elif variant == "mha_d128" and -(-seq // 256) * heads * bsz < 256:
-            # 256-row blocks leave CUs idle: 128-row blocks of the same softmax
-            # (B1 H16 S2048 49.9 -> 43.4 us, B1 H8 S512 16.7 -> 13.6 us)
+        elif variant == "mha_d128" and -(-seq // 128) * heads * bsz <= 256:
+            # 256-row blocks leave CUs idle: 128-row blocks of the same softmax, while there is
+            # at most one per CU (B1 H16 S2048 49.9 -> 43.4 us, B1 H8 S512 16.7 -> 13.6 us;
+            # 336 blocks, B6 H8 S896: 26.5 -> 27.6 us)
             variant = "mha_d128_w4"
     handle = kernels.handle(variant)
     kv_tile = next(o for o in _loops(handle.kernel)).tile_size
@@ -498,7 +499,8 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     each query head's fp32 dK / dV contribution into ``workspace`` (fp32, at
     least ``2 * B * H * S * D`` elements, allocated if omitted) and a HIP
     reduction sums the ``H / H_kv`` contributions of every key/value head
-    into bf16 ``dK`` / ``dV``.  Two WarpIR kernels run
+    into bf16 ``dK`` / ``dV``.  Two WarpIR kernels (or, for small launches,
+    their hand-written split forms, ``attn_bwd_split.hip``) run
     on the current stream: the query-major dQ kernel, which also writes
     ``Dv = rowsum(dO * O)`` (into ``dvec``, fp32 ``[B, H, S]``, allocated if
     omitted) and the LSE in log2 units, and the key-major dK/dV kernel, which
@@ -546,6 +548,10 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     # (handle, arguments, views) of each launch in order
     launches = [(kernels.handle(f"mha_bwd_dq_prep_d{d}{sfx}"), dq_args, None),
                 (kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}"), dkdv_args, views)]
+    if planned and hr == 1 and _split_bwd_fits(bsz, heads, seq, q, k, v, do):
+        _attention_bwd_split(launches, causal, rec, dvec)
+        _backward_plans.add(1 if causal else 0, rec, dq, dk, dv)
+        return dq, dk, dv
     for handle, args, _ in launches:
         handle(**args)
     reductions = []
@@ -559,6 +565,41 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
                     [(type(args).partials.offset, rec.slot(workspace), off), (type(args).out.offset, rec.slot(grad), 0)])
         _backward_plans.add(1 if causal else 0, rec, dq, dk, dv)
     return dq, dk, dv
+
+
+def _split_bwd_fits(bsz: int, heads: int, seq: int, *loaded) -> bool:
+    """Whether the backward goes to the split kernels (``attn_bwd_split.hip``,
+    32 rows per program, one program per CU at a time).  dQ + dK/dV in us,
+    tiled -> split: B1 H8 S512 D64 14.9 + 17.5 -> 8.0 + 8.3 (128 programs), S1024
+    24.3 + 29.3 -> 11.3 + 12.5 (256); at 512 programs S2048 D64 43.5 + 53.1 ->
+    32.5 + 37.9, causal 42.3 + 64.4 -> 23.2 + 24.7, H16 S1024 D128 33.1 + 37.4 ->
+    33.5 + 35.6.  Their lane offsets are 32-bit."""
+    return 0 < bsz * heads * (seq // 32) <= 512 and all(0 <= t.stride(2) < 1 << 23 for t in loaded)
+
+
+_split_bwd_kernels: dict = {}
+
+
+def _attention_bwd_split(launches, causal: bool, rec: Recording, dvec) -> None:
+    """Launch the split dQ and dK/dV kernels on the arguments of the tiled
+    kernels in *launches*, which validate and pack them, and record them."""
+    import torch
+
+    from warpir_amd.runtime import RawKernel
+
+    stream = torch.cuda.current_stream(dvec.device).cuda_stream
+    for part, (handle, args, _) in zip(("dq", "dkdv"), launches):
+        bsz, heads, seq, d = args["Q"].shape
+        name = f"wir_attn_{part}_split_d{d}" + ("_causal" if causal else "")
+        kernel = _split_bwd_kernels.get(name)
+        if kernel is None:
+            kernel = _split_bwd_kernels.setdefault(name, RawKernel("attn_bwd_split.hsaco", name))
+        packed = handle.pack(args)[0]
+        grid, block = (seq // 32, heads, bsz), (256, 1, 1)
+        kernel.launch(grid, block, packed, stream=stream)
+        rec.raw(kernel._function, grid, block, packed,
+                [(getattr(handle.args_type, f).offset, rec.slot(x), 0) for f, x in args.items()
+                 if isinstance(x, torch.Tensor)])
 
 
 _group_reduce_kernel = None
