@@ -134,3 +134,14 @@ def test_tables_are_bounded_and_calls_from_threads_agree(gpu, fresh):
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not bad
+
+
+def test_a_causal_flag_that_is_no_truth_value_stays_refused_beside_a_plan(gpu, fresh):
+    q, k, v = (seeded_normal((1, 2, 128, 64), s).cuda() for s in range(3))
+    for causal in (False, True):
+        for _ in range(2):
+            o, _ = api.attention_forward(q, k, v, causal=causal)
+        assert torch.equal(api.attention_forward(q, k, v, causal=int(causal))[0], o)
+    for causal in (None, 2, "yes"):
+        with pytest.raises(ValueError, match="no kernel variant"):
+            api.attention_forward(q, k, v, causal=causal)

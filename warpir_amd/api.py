@@ -393,7 +393,7 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     """
     import torch
 
-    planned = variant is None
+    planned = variant is None and type(causal) in (bool, int) and 0 <= causal <= 1   # others are refused below
     if planned:
         done = _forward_plans.run(1 if causal else 0, q, k, v, out, lse)
         if done is not None:
