@@ -303,7 +303,7 @@ def _bwd_inputs():
 
 
 def _extra_fa_bwd(steps: int, warmup: int):
-    """FlashAttention backward at the config-4 shape (prep + dQ + dK/dV kernels)."""
+    """FlashAttention backward at the config-4 shape (the dQ kernel, which also writes Dv and the log2 LSE, and dK/dV)."""
     import torch
 
     from warpir_amd import api
@@ -316,7 +316,7 @@ def _extra_fa_bwd(steps: int, warmup: int):
     tf = api.attention_backward_flops(bsz, heads, seq, d) / (ms * 1e-3) / 1e12
     return {"fa_bwd_b16_h16_s4096_d128": {
         "ms": ms, "tflops": tf, "frac_mfma": tf / PEAK_BF16_TFLOPS,
-        "kernels": ["mha_bwd_prep_d128", "mha_bwd_dq_d128", "mha_bwd_dkdv_d128"],
+        "kernels": ["mha_bwd_dq_prep_d128", "mha_bwd_dkdv_d128"],
         "flops": "10*B*H*S^2*D (the five S x S x D products); the kernels run seven (dQ recomputes S and dP)"}}
 
 
@@ -339,7 +339,7 @@ def _extra_fa_causal_d128(steps: int, warmup: int):
     tf = api.attention_backward_flops(bsz, heads, seq, d, causal=True) / (ms * 1e-3) / 1e12
     out["fa_bwd_causal_b16_h16_s4096_d128"] = {
         "ms": ms, "tflops": tf, "frac_mfma": tf / PEAK_BF16_TFLOPS,
-        "kernels": ["mha_bwd_prep_d128", "mha_bwd_dq_d128_causal", "mha_bwd_dkdv_d128_causal"],
+        "kernels": ["mha_bwd_dq_prep_d128_causal", "mha_bwd_dkdv_d128_causal"],
         "flops": "5*B*H*S^2*D (the five products, halved by the causal mask)"}
     return out
 
