@@ -422,7 +422,9 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     if lse is None:
         lse = rec.alloc(torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device))
     args = dict(Q=q, K=k, V=v, N=seq, O=out, L=lse)
-    if planned and _split_kv_fits(bsz, heads, seq, causal, k, v):
+    if (planned and _split_kv_fits(bsz, heads, seq, causal, k, v)
+            and out.shape == q.shape and lse.shape == (bsz, heads, seq)):
+        # (the tiled kernels' grid covers destinations of other shapes: what does not fit is dropped)
         _attention_split_kv(handle, args, hr, causal, rec)
         return out, lse
     if any(v_.name == "HR" for v_ in handle.kernel.inputs):
@@ -548,7 +550,8 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     # (handle, arguments, views) of each launch in order
     launches = [(kernels.handle(f"mha_bwd_dq_prep_d{d}{sfx}"), dq_args, None),
                 (kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}"), dkdv_args, views)]
-    if planned and hr == 1 and _split_bwd_fits(bsz, heads, seq, q, k, v, do):
+    if (planned and hr == 1 and _split_bwd_fits(bsz, heads, seq, q, k, v, do)
+            and all(g.shape == q.shape for g in (dq, dk, dv)) and dvec.shape == lse.shape):   # as in the forward
         _attention_bwd_split(launches, causal, rec, dvec)
         _backward_plans.add(1 if causal else 0, rec, dq, dk, dv)
         return dq, dk, dv

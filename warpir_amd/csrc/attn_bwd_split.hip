@@ -10,7 +10,7 @@
 // barrier); the fp32 partial sums are added through LDS in wave order and
 // rounded once.  Device time, tiled -> here: B1 H8 S512 D64 dQ 14.9 -> 8.0 us,
 // dK/dV 17.5 -> 8.3 us; S1024 D128 31.9 -> 17.7 and 36.8 -> 19.9 us.
-#include "wir_cdna4.h"
+#include "wir_split.h"
 
 namespace {
 
@@ -83,7 +83,7 @@ __device__ __forceinline__ void put_partial(lds_float* part, const wir::RTile<32
 template <int D>
 __device__ __forceinline__ void store_sum(const lds_float* part, const wir::gl<bf16>& g, int b, int h, int row0,
                                           float scale) {
-  bf16* base = g.data + (long long)b * g.sb + (long long)h * g.sd;
+  const wir::RowStore out(g, b, h);
 #pragma unroll
   for (int it = 0; it < ROWS * (D / 8) / (WAVES * 64); ++it) {
     const int idx = it * WAVES * 64 + threadIdx.x;
@@ -101,11 +101,10 @@ __device__ __forceinline__ void store_sum(const lds_float* part, const wir::gl<b
         acc[4 + j] += hi[j];
       }
     }
-    if (row0 + row >= g.r) continue;
     bf16x8 v;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (bf16)(acc[j] * scale);
-    *(bf16x8*)(base + (long long)(row0 + row) * g.sr + ch * 8) = v;
+    out.put8(g, row0 + row, ch * 8, v);
   }
 }
 

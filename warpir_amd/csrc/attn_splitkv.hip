@@ -21,7 +21,7 @@
 // The softmax is the exact online one (a running maximum per wave, fp32 sums,
 // probabilities rounded to bf16 for the second product), so its error is that
 // of the exact tiled kernels; the merge rescales in fp32 and rounds O once.
-#include "wir_cdna4.h"
+#include "wir_split.h"
 
 namespace {
 
@@ -173,8 +173,9 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
   }
   wir::barrier();
 
-  bf16* ob = args.O.data + (long long)b * args.O.sb + (long long)h * args.O.sd;
+  const wir::RowStore out(args.O, b, h);
   float* lb = args.L.data + (long long)b * args.L.sb + (long long)h * args.L.sd;
+  const int lse_rows = (unsigned)b < (unsigned)args.L.b && (unsigned)h < (unsigned)args.L.d ? args.L.r : 0;
 #pragma unroll
   for (int it = 0; it < ROWS * (D / 8) / (WAVES * 64); ++it) {
     const int idx = it * WAVES * 64 + threadIdx.x;
@@ -199,13 +200,12 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
         acc[4 + j] += f * hi[j];
       }
     }
-    if (row0 + row >= args.O.r) continue;
     const float inv = 1.0f / sum;
     bf16x8 v;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (bf16)(acc[j] * inv);
-    *(bf16x8*)(ob + (long long)(row0 + row) * args.O.sr + ch * 8) = v;
-    if (ch == 0 && row0 + row < args.L.r)
+    out.put8(args.O, row0 + row, ch * 8, v);
+    if (ch == 0 && row0 + row < lse_rows)
       lb[(long long)(row0 + row) * args.L.sr] = (top * c + __builtin_amdgcn_logf(sum)) * kLn2;
   }
 }
