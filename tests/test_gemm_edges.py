@@ -92,6 +92,15 @@ def test_clamped_body_is_emitted_for_plain_gemms_only():
         assert "wir_body(wir::bool_tag<true, true>" not in CDNA4Lowerer(target).lower(kernels.kernel(name))
 
 
+@pytest.mark.parametrize("name", VARIANTS)
+def test_clamped_body_needs_results_that_end_with_the_operands(name):
+    """A destination that goes on past A's rows or B's columns has zeros there,
+    which clamped lanes do not give."""
+    line = next(ln for ln in _source(name).split("\n") if "else if (" in ln and "clamped" in ln)
+    assert "::clampable<1>(globals.A, globals.C_global.r)" in line
+    assert "::clampable<2>(globals.B, globals.C_global.c)" in line
+
+
 def test_only_a_loop_without_shifted_rings_has_a_checked_copy():
     """A ring that runs behind the loop loads its last tiles in drain steps,
     which have no checked copy: its reduction extent must be whole tiles."""

@@ -58,6 +58,22 @@ def test_ragged_gemm_keeps_infinities_in_their_row_and_column(gpu, variant):
     assert rel_err(c[:m - 1, :n - 1], gemm_ref(a[:m - 1], b[:, :n - 1])) <= TOL
 
 
+@pytest.mark.parametrize("variant", EDGE_VARIANTS)
+@pytest.mark.parametrize("rows,cols", [(28, 0), (0, 24), (300, 264), (-5, 0), (0, -8)])
+def test_destination_of_another_shape_has_zeros_past_the_product(gpu, variant, rows, cols):
+    """Clamped lanes feed only results past the end of A or B: where C goes on
+    there, its elements are zero, and a smaller C drops what does not fit."""
+    m, n, k = 100, 136, 264
+    a, b = seeded_normal((m, k), 6), seeded_normal((k, n), 7)
+    c = torch.full((m + rows, n + cols), -7.0, dtype=torch.bfloat16, device="cuda")
+    kernels.handle(variant)(A=a.cuda(), B=b.cuda(), N=k, C_global=c)
+    want = torch.zeros(m + max(rows, 0), n + max(cols, 0))
+    want[:m, :n] = gemm_ref(a, b)
+    want = want[:m + rows, :n + cols]
+    assert rel_err(c.cpu(), want) <= TOL
+    assert bool((c.cpu()[m:] == 0).all()) and bool((c.cpu()[:, n:] == 0).all())
+
+
 @pytest.mark.parametrize("variant", ["gemm_64_k64", "gemm_64x128_k64"])
 @pytest.mark.parametrize("m,n,k", [(64, 128, 64), (128, 128, 256), (192, 256, 320), (1024, 1024, 1024)])
 def test_small_tiles_match_the_256_tile_bit_for_bit(gpu, variant, m, n, k):

@@ -276,10 +276,13 @@ struct Loader {
     return g.r % Tile::ROWS == 0 && g.c % Tile::COLS == 0 && (long long)Tile::ROWS * g.sr < (1ll << 30);
   }
 
-  // Whether `g` suits the clamped form: whole 16-byte chunks per row, and a
-  // row pitch that fits the 32-bit lane offsets.
-  static __device__ __forceinline__ bool clampable(const gl<bf16>& g) {
-    return g.c % 8 == 0 && (long long)Tile::ROWS * g.sr < (1ll << 30);
+  // Whether `g` suits the clamped form: whole 16-byte chunks per row, a row
+  // pitch that fits the 32-bit lane offsets, and no result row (CLAMP 1) or
+  // column (2) stored past its end (`stored` of them are; a destination may
+  // be larger than the product, and has zeros there).
+  template <int CLAMP>
+  static __device__ __forceinline__ bool clampable(const gl<bf16>& g, int stored) {
+    return g.c % 8 == 0 && (long long)Tile::ROWS * g.sr < (1ll << 30) && stored <= (CLAMP == 1 ? g.r : g.c);
   }
 };
 

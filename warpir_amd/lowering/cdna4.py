@@ -1308,7 +1308,7 @@ class CDNA4Lowerer:
         program id indexes, clamped in the WIR_EDGE body (``wir::Loader``)."""
         if not self._edge or not isinstance(op, TMALoadBufOp):
             return ""
-        dims = [k for k, c in ((1, op.coords[2]), (2, op.coords[3])) if isinstance(c, Value) and c.name in _GRID]
+        dims = _grid_dims(op)
         return f", WIR_EDGE ? {dims[0]} : 0" if len(dims) == 1 else ""
 
     def _load_call(self, op, fn: str, ptr: str, key: str) -> str:
@@ -2996,8 +2996,9 @@ class CDNA4Lowerer:
         such body.  It is the in-bounds body for extents that are no
         multiples of the tile: a dimension that a program id indexes needs
         only the program's tile origin inside (its lanes clamp to the last
-        row or chunk), the loop's last tile may be cut (``_checked_tail``),
-        and the other coordinates are bounded as in ``_in_bounds_checks``.
+        row or chunk) and no result stored past its end, the loop's last tile
+        may be cut (``_checked_tail``), and the other coordinates are bounded
+        as in ``_in_bounds_checks``.
         Launches that were in bounds as a whole take the aligned body."""
         ops = list(_walk(kernel.body))
         loops = [op for op in kernel.body if isinstance(op, ForOp)]
@@ -3027,7 +3028,12 @@ class CDNA4Lowerer:
                 continue
             g = f"globals.{_cname(op.source.name)[2:]}"
             sub = op.source.type.sub_tile_type
-            conds.append(f"wir::Loader<{self.stile(self.resolve(op.buf.name))}, {self.geo.nw}>::clampable({g})")
+            dims = _grid_dims(op)
+            stored = self._stored_extent(kernel, op, dims[0]) if len(dims) == 1 else None
+            if stored is None:
+                return []
+            conds.append(f"wir::Loader<{self.stile(self.resolve(op.buf.name))}, {self.geo.nw}>"
+                         f"::clampable<{dims[0]}>({g}, {stored})")
             for c, unit, dim in zip(op.coords, (1, 1, sub.rows, sub.cols), "bdrc"):
                 if isinstance(c, int):
                     first[f"{g}.{dim}"] = max(first.get(f"{g}.{dim}", 0), (c + 1) * unit)
@@ -3041,6 +3047,23 @@ class CDNA4Lowerer:
                     return []
         conds += [f"{v} <= {e}" for e, v in first.items()]
         return list(dict.fromkeys(conds))
+
+    def _stored_extent(self, kernel: Kernel, load, dim: int) -> Optional[str]:
+        """The extent (C++ text) in which the kernel's stores run along the
+        grid index of *load*'s dimension *dim* (1 = rows, 2 = columns), or
+        None where their tiles are not the load's along it."""
+        sub = load.source.type.sub_tile_type
+        unit = sub.rows if dim == 1 else sub.cols
+        out = []
+        for op in _walk(kernel.body):
+            if isinstance(op, TMAStoreOp):
+                dsub = op.dest.type.sub_tile_type
+                for c, size, name in ((op.coords[2], dsub.rows, "r"), (op.coords[3], dsub.cols, "c")):
+                    if isinstance(c, Value) and c.name == load.coords[1 + dim].name:
+                        if size != unit:
+                            return None
+                        out.append(f"globals.{_cname(op.dest.name)[2:]}.{name}")
+        return out[0] if len(out) == 1 else None
 
     def _wave_tile(self) -> RegTileType:
         """The register tile shape that sets the wavefront slices: the first
@@ -3184,6 +3207,11 @@ class _Sim:
 # helpers
 # ----------------------------------------------------------------------
 _GRID = ("blockIdx.x", "blockIdx.y", "blockIdx.z")
+
+
+def _grid_dims(op) -> List[int]:
+    """The dimensions of a tile load (1 = rows, 2 = columns) that a program id indexes."""
+    return [k for k, c in ((1, op.coords[2]), (2, op.coords[3])) if isinstance(c, Value) and c.name in _GRID]
 
 
 def _buffer_form(kernel: Kernel) -> bool:
