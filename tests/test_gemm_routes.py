@@ -1,0 +1,53 @@
+"""api.gemm's choice of a kernel, on the CPU: kernels and split-K replaced by
+recorders."""
+import pytest
+import torch
+
+from warpir_amd import api, kernels
+
+
+def _bf16(*shape):
+    return torch.zeros(*shape, dtype=torch.bfloat16)
+
+
+@pytest.fixture
+def taken(monkeypatch):
+    log = []
+
+    class Handle:
+        def __init__(self, name):
+            self.name = name
+
+        def __call__(self, **kw):
+            log.append(self.name)
+
+    monkeypatch.setattr(kernels, "handle", Handle)
+    monkeypatch.setattr(api, "gemm_split_k", lambda a, b, out=None, workspace=None: log.append("split-K") or out)
+    return log
+
+
+# (m, n, k) that split-K takes by estimate: long K with M > 128, and with M <= 128 but fewer than four slices
+SPLIT = [(200, 1024, 8192), (16, 8192, 6336)]
+
+
+@pytest.mark.parametrize("m,n,k", SPLIT)
+def test_destinations_of_another_shape_keep_the_tiled_kernels(taken, m, n, k):
+    assert api.gemm_variant(m, n, k) == api.SPLITK_GEMM_VARIANT
+    a, b = _bf16(m, k), _bf16(k, n)
+    api.gemm(a, b, out=_bf16(m, n))
+    for shape in ((m - 8, n), (m + 8, n), (m, n + 64), (1, m, n)):
+        api.gemm(a, b, out=_bf16(*shape))
+    assert taken == ["split-K", *[api._gemm_route(m, n, k)[1]] * 4]
+
+
+def test_short_m_of_long_k_still_refuses_them():
+    """Where M <= 128 has four slices every dense call went to split-K, which
+    refuses a destination of another shape, and so it does where the estimate
+    now prefers a tiled kernel."""
+    refused = 0
+    for m, n, k in ((64, 8192, 8192), (64, 1024, 512), (8, 256, 1024), (128, 512, 256)):
+        assert api.splitk_count(m, n, k) >= 4
+        refused += api.gemm_variant(m, n, k) != api.SPLITK_GEMM_VARIANT
+        with pytest.raises(ValueError, match="out must be"):
+            api.gemm(_bf16(m, k), _bf16(k, n), out=_bf16(m + 8, n))
+    assert refused

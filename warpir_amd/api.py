@@ -337,18 +337,23 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
     if out is None:
         out = rec.alloc(torch.empty(m, n, dtype=torch.bfloat16, device=a.device))
     if variant is None:
-        variant = gemm_variant(m, n, k)
+        variant, tiled = _gemm_route(m, n, k)
+        short = m <= 128 and splitk_count(m, n, k) >= 4
         if workspace is not None:
             # a workspace is the caller's choice of split-K wherever M <= 128 has at least four
             # slices, and is not read elsewhere
-            if m <= 128 and splitk_count(m, n, k) >= 4:
+            if short:
                 variant = SPLITK_GEMM_VARIANT
             else:
                 workspace = None
-        if variant == SPLITK_GEMM_VARIANT and not _splitk_operands_ok(a, b, out):
+        if not _splitk_operands_ok(a, b, out):
             # the split-K entry points take dense operands only; the tiled
             # kernel reads row-strided views through the globals' row stride
-            variant = _gemm_route(m, n, k)[1]
+            variant = tiled
+        elif tuple(out.shape) != (m, n):
+            # split-K, which short M of long K always took, refuses it; the tiled kernels
+            # drop what does not fit and write zeros past the product
+            variant = SPLITK_GEMM_VARIANT if short else tiled
     if variant == SPLITK_GEMM_VARIANT:
         splits = splitk_count(m, n, k)
         if planned and a.is_cuda:
