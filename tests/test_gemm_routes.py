@@ -51,3 +51,17 @@ def test_short_m_of_long_k_still_refuses_them():
         with pytest.raises(ValueError, match="out must be"):
             api.gemm(_bf16(m, k), _bf16(k, n), out=_bf16(m + 8, n))
     assert refused
+
+
+@pytest.mark.parametrize("m,n,k", SPLIT)
+def test_a_workspace_that_split_k_does_not_take_keeps_the_tiled_kernels(taken, m, n, k):
+    """A call with a workspace allocates no partials of its own."""
+    assert not (m <= 128 and api.splitk_count(m, n, k) >= 4)
+    api.gemm(_bf16(m, k), _bf16(k, n), out=_bf16(m, n), workspace=torch.zeros(8))
+    assert taken == [api._gemm_route(m, n, k)[1]]
+
+
+def test_a_workspace_asks_for_split_k(taken):
+    assert api.gemm_variant(64, 1024, 512) != api.SPLITK_GEMM_VARIANT
+    api.gemm(_bf16(64, 512), _bf16(512, 1024), workspace=torch.zeros(8 * 64 * 1024))
+    assert taken == ["split-K"]

@@ -3,9 +3,9 @@
 These play the role of the reference harness's launch wrappers
 (``launch_gemm(A, B, C)``, ``tests/test_modal_gpu.py:24-50``;
 ``launch_attention(Q, K, V, O)``, ``tests/test_modal_attention.py:25-39``):
-validate shapes, allocate nothing but the outputs the caller did not
-pass, and launch the WarpIR-generated HIP kernel through the C ABI on the
-current stream.  They raise on a CPU tensor or a missing GPU; there is no
+validate shapes, allocate nothing but the outputs and fp32 workspaces the
+caller did not pass, and launch the WarpIR-generated HIP kernel through the
+C ABI on the current stream.  They raise on a CPU tensor or a missing GPU; there is no
 fallback implementation.
 """
 from __future__ import annotations
@@ -316,9 +316,11 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
 
     The variant follows ``gemm_variant``: 256x256 tiles for outputs that fill
     the chip with them, smaller tiles for others, split-K for few tiles and
-    long K (``workspace`` as in ``gemm_split_k``, taken for M <= 128).  An empty output (M or
-    N = 0) launches nothing; K = 0 gives zeros (the kernel's loop runs no
-    step and its tile loads read the zero page).
+    long K.  ``workspace`` (as in ``gemm_split_k``) asks for split-K where
+    M <= 128 has at least four slices and is not read elsewhere; a call that
+    passes it and ``out`` allocates nothing.  An empty output (M or N = 0)
+    launches nothing; K = 0 gives zeros (the kernel's loop runs no step and
+    its tile loads read the zero page).
     """
     import torch
 
@@ -340,12 +342,9 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
         variant, tiled = _gemm_route(m, n, k)
         short = m <= 128 and splitk_count(m, n, k) >= 4
         if workspace is not None:
-            # a workspace is the caller's choice of split-K wherever M <= 128 has at least four
-            # slices, and is not read elsewhere
-            if short:
-                variant = SPLITK_GEMM_VARIANT
-            else:
-                workspace = None
+            # the caller's choice of split-K there; elsewhere it is not read, and no partials are
+            # allocated beside it
+            variant = SPLITK_GEMM_VARIANT if short else tiled
         if not _splitk_operands_ok(a, b, out):
             # the split-K entry points take dense operands only; the tiled
             # kernel reads row-strided views through the globals' row stride
