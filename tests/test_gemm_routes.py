@@ -65,3 +65,13 @@ def test_a_workspace_asks_for_split_k(taken):
     assert api.gemm_variant(64, 1024, 512) != api.SPLITK_GEMM_VARIANT
     api.gemm(_bf16(64, 512), _bf16(512, 1024), workspace=torch.zeros(8 * 64 * 1024))
     assert taken == ["split-K"]
+
+
+@pytest.mark.parametrize("m,n,k", [(128, 16384, 8192), (128, 16384, 16384), (64, 8192, 8192), (200, 1024, 8192)])
+def test_operands_that_split_k_does_not_take_get_the_fastest_tile(m, n, k):
+    """Strided operands of a product that split-K would take go to the tiled
+    variant with the smallest estimate, for short M too."""
+    route, fallback = api._gemm_route(m, n, k)
+    assert route == api.SPLITK_GEMM_VARIANT
+    est = {v: api._tiled_estimate(c, m, n, k) for v, c in api._TILE_COST.items()}
+    assert est[fallback] == min(est.values())

@@ -26,7 +26,7 @@ _forward_plans = Plans("attention_forward")
 _backward_plans = Plans("attention_backward")
 
 GEMM_VARIANT = "gemm_256_k64"
-SKINNY_GEMM_VARIANT = "gemm_64_k64"       # short M, long K, operands that split-K does not take
+SKINNY_GEMM_VARIANT = "gemm_64_k64"       # short M and few columns: what the estimate gives there
 MID_GEMM_VARIANT = "gemm_128_k64"         # K unknown, fewer 256x256 tiles than CUs: 128x128 tiles
 
 # Time of one product on the 256 CUs of an MI355X, in microseconds, as a
@@ -95,11 +95,14 @@ def gemm_variant(m: int, n: int, k: Optional[int] = None) -> str:
 
 @functools.lru_cache(maxsize=1024)
 def _gemm_route(m: int, n: int, k: int) -> Tuple[str, str]:
-    """(variant, variant for operands that split-K does not take)."""
+    """(variant, variant for operands that split-K does not take: the tile with
+    the smallest estimate.  Row-strided A, us: 128x16384x8192 gemm_128x64_k64
+    74.8 against gemm_64_k64's 95.3, 128x8192x8192 the other way, 67.4 and
+    48.7)."""
     tiled, est = min(((v, _tiled_estimate(c, m, n, k)) for v, c in _TILE_COST.items()), key=lambda x: x[1])
     splits = splitk_count(m, n, k)
     if splits > 1 and _splitk_estimate(m, n, k, splits) < est:
-        return SPLITK_GEMM_VARIANT, SKINNY_GEMM_VARIANT if m <= 128 else tiled
+        return SPLITK_GEMM_VARIANT, tiled
     return tiled, tiled
 
 
