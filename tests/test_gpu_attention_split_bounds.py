@@ -7,7 +7,7 @@ import torch
 from oracle.torch_ref import attention_bwd_ref, attention_ref, rel_err, seeded_normal
 from tests.conftest import announce
 from warpir_amd import api, kernels
-from warpir_amd.plans import Recording
+from warpir_amd.plans import NO_RECORDING
 
 pytestmark = pytest.mark.gpu
 
@@ -64,7 +64,8 @@ def test_forward_drops_what_does_not_fit(gpu, d, causal, shape):
                              (128, True): "mha_d128_causal"}[d, causal])
 
     def split():   # the split kernel itself, which no route gives such destinations
-        api._attention_split_kv(handle, dict(Q=q, K=k, V=v, N=S, O=out, L=lse), 1, causal, Recording(q, k, v, out, lse))
+        args = dict(Q=q, K=k, V=v, N=S, O=out, L=lse)
+        api._attention_split_kv(handle.pack(args), args, q.shape, 1, causal, NO_RECORDING)
 
     for launch in (lambda: api.attention_forward(q, k, v, causal=causal, out=out, lse=lse),) * 2 + (split,):
         big.fill_(MARK), lbig.fill_(MARK)
@@ -96,9 +97,7 @@ def test_backward_drops_what_does_not_fit(gpu, d, causal, shape):
                  dict(Q=q, K=k, V=v, dO=do, L2=lse2, Dv=dvec, N=S, dK=grads[1], dV=grads[2]), None)]
 
     def split():
-        rec = Recording(q, k, v, o, lse, do, *grads, dvec)
-        rec.alloc(lse2)
-        api._attention_bwd_split(launches, causal, rec, dvec)
+        api._attention_bwd_split(launches, causal, NO_RECORDING, dvec)
 
     for launch in (lambda: api.attention_backward(q, k, v, o, lse, do, *grads, causal=causal),) * 2 + (split,):
         for big in bigs:

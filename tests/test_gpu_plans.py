@@ -145,3 +145,111 @@ def test_a_causal_flag_that_is_no_truth_value_stays_refused_beside_a_plan(gpu, f
     for causal in (None, 2, "yes"):
         with pytest.raises(ValueError, match="no kernel variant"):
             api.attention_forward(q, k, v, causal=causal)
+
+
+class _Subclass(torch.Tensor):
+    pass
+
+
+def _plannable(*tensors):
+    """What an empty table says of a call with these tensors."""
+    r = native().run(native().table(), 0, *tensors)
+    assert r is None or r is False
+    return r is False
+
+
+def _in_mode(mode, *tensors):
+    with mode:
+        return _plannable(*tensors)
+
+
+def test_calls_that_can_have_no_plan(gpu, fresh):
+    """Active torch-function and dispatch modes, functorch and Python wrappers,
+    subclasses, conjugate or misaligned or empty tensors, one tensor twice."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    a, b = seeded_normal((64, 64), 0).cuda(), seeded_normal((64, 64), 1).cuda()
+    plan = _plannable
+    assert plan(a, b, None) and plan(a, torch.nn.Parameter(b)) and plan(a, b.clone().requires_grad_())
+    for mode in (Function(), Dispatch(), torch.device("cuda")):
+        assert not _in_mode(mode, a, b)
+    assert plan(a, b)
+    assert not plan(a, a) and not plan(a, b[:0]) and not plan(a, a.cpu()) and not plan(None, None)
+    assert not plan(a, a.flatten()[1:-7].view(8, 511)) and not plan(a, a.as_subclass(_Subclass))
+    assert not plan(a, torch._neg_view(b.float())) and not plan(a, b.to_sparse())
+    seen = []
+    torch.func.vmap(lambda x: seen.append(plan(x, b)) or x)(a[None])
+    torch.func.grad(lambda x: seen.append(plan(x, b)) or x.sum())(a.float())
+    assert seen == [False, False]
+    for mode in (Function(), torch.device("cuda")):   # refused by a table that holds the plan, too
+        ref = api.gemm(a, b)
+        with mode:
+            assert torch.equal(api.gemm(a, b), ref)
+    assert torch.equal(api.gemm(a, b.as_subclass(_Subclass)), ref)
+    assert _count(api._gemm_plans) == 1
+
+
+def test_calls_without_a_plan_pack_their_arguments_once(gpu, fresh, monkeypatch):
+    """What a call without plans costs: validated and packed on its first call,
+    from the handles' caches on later ones, and nothing packed for a plan."""
+    from warpir_amd.runtime import KernelHandle
+
+    packed, real = [], KernelHandle.pack
+    monkeypatch.setattr(KernelHandle, "pack", lambda self, args: packed.append(self) or real(self, args))
+
+    def twice(call, launches):
+        for n in (launches, 0):
+            packed.clear()
+            call()
+            assert len(packed) == n
+
+    x = seeded_normal((64, 64), 0).cuda()
+    y = torch.empty_like(x)
+    a, b = seeded_normal((64, 4096), 1).cuda(), seeded_normal((4096, 256), 2).cuda()
+    twice(lambda: api.gemm(x, x, out=y), 1)
+    assert api.gemm_variant(64, 256, 4096) == api.SPLITK_GEMM_VARIANT
+    for heads in (2, 600):   # the split and the tiled kernels
+        q, k, v, do, o, dq, dk, dv = (seeded_normal((1, heads, 128, 64), s).cuda() for s in range(8))
+        flat = torch.empty(heads * 128 + 1, device="cuda")
+        lse, dvec = flat[1:].view(1, heads, 128), torch.empty(1, heads, 128, device="cuda")   # lse: 4-byte aligned
+        twice(lambda: api.attention_forward(q, k, v, out=o, lse=lse), 1)
+        # (its log2 LSE is allocated on every call, where the allocator gives the same memory again)
+        twice(lambda: api.attention_backward(q, k, v, o, lse, do, dq, dk, dv, dvec), 2)
+    out, z = torch.empty(64, 256, dtype=torch.bfloat16, device="cuda"), torch.empty_like(x)
+    with torch.device("cuda"):
+        twice(lambda: api.gemm(a, b, out=out), 0)
+        twice(lambda: api.gemm(x, y, out=z), 1)
+    assert all(_count(p) == 0 for p in (api._gemm_plans, api._forward_plans, api._backward_plans))
+    packed.clear()
+    api.gemm(x, y)   # a call that leaves a plan packs once as well
+    assert len(packed) == 1 and _count(api._gemm_plans) == 1
+
+
+def test_a_full_table_keeps_part_of_more_signatures_than_it_holds(gpu, fresh, monkeypatch):
+    b = seeded_normal((8, 8), 1).cuda()
+    rows = [seeded_normal((m, 8), m).cuda() for m in range(1, 321)]
+    want = [gemm_ref(a.cpu(), b.cpu()) for a in rows]
+    missed, real = [], api._gemm_plans.run
+
+    def run(*args):
+        done, got = real(*args)
+        missed.extend([1] * (not done))
+        return done, got
+
+    monkeypatch.setattr(api._gemm_plans, "run", run)
+    for _ in range(4):
+        missed.clear()
+        for a, w in zip(rows, want):
+            assert rel_err(api.gemm(a, b).cpu(), w) <= 1e-2
+        assert _count(api._gemm_plans) == 256
+    # 256 of 320 held: a random replacement finds most of them, dropping the oldest or all would find none
+    assert len(missed) < 200

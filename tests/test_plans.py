@@ -25,3 +25,13 @@ def test_recording_finds_a_tensor_by_its_argument():
     rec = plans.Recording(a, None, b)
     rec.alloc(out)
     assert [rec.slot(x) for x in (a, b, out)] == [0, 2, 3]
+
+
+@pytest.mark.skipif(not os.path.exists(os.path.join(PKG_DIR, "_wir_plans.so")), reason="not built")
+def test_cpu_calls_record_nothing():
+    t = torch.zeros(8, 8, dtype=torch.bfloat16)
+    for loaded in (False, True):
+        if loaded:
+            plans.native()
+        done, rec = plans.Plans("x").run(0, t, t.clone())
+        assert not done and rec is plans.NO_RECORDING and not rec and rec.alloc(t) is t

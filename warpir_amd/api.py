@@ -10,12 +10,14 @@ fallback implementation.
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import math
 from typing import Optional, Tuple
 
 from warpir_amd import kernels
-from warpir_amd.plans import Plans, Recording
+from warpir_amd.plans import NO_RECORDING, Plans, Recording
+from warpir_amd.runtime import GL, RawKernel
 
 # Plans of the calls below, by flags: gemm 0; attention_forward and
 # attention_backward the causal bit.  A stream of calls, before -> after: gemm
@@ -106,6 +108,12 @@ def _gemm_route(m: int, n: int, k: int) -> Tuple[str, str]:
     return tiled, tiled
 
 
+@functools.lru_cache(maxsize=1024)
+def _always_split(m: int, n: int, k: int) -> bool:
+    """Short M of long K: what goes to split-K without an estimate."""
+    return m <= 128 and splitk_count(m, n, k) >= 4
+
+
 # 128x128 tiles, 64-deep K steps; kernel_pass sizes the rings per operand:
 # B (streamed from HBM) seven slots loaded six steps ahead, A (the row panel
 # every program re-reads from L2) three slots, filling 160 KiB of LDS
@@ -175,8 +183,6 @@ def _splitk_functions(variant: str):
     first use of a variant checks that its launch geometry is the one the C
     ABI's split-K entry points build (128x128 tiles, 256 threads, slices on
     blockIdx.z)."""
-    from warpir_amd.runtime import RawKernel
-
     global _reduce_kernel
     h = kernels.handle(variant)
     if variant not in _splitk_checked:
@@ -205,8 +211,6 @@ def gemm_split_k(a, b, out=None, splits: Optional[int] = None, workspace=None, v
     fp32 tensor of at least ``splits * M * N`` elements (allocated if
     omitted); ``variant`` names a split-K kernel variant (default
     ``SPLITK_GEMM_VARIANT``)."""
-    import ctypes
-
     import torch
 
     from warpir_amd.runtime import check, library
@@ -271,8 +275,6 @@ def gemm_split_k_noalloc(a, b, out, splits: Optional[int] = None, stream=None):
     Raises ``HipError`` when ``splits * M * N`` exceeds the scratch
     (``NOALLOC_SCRATCH_FLOATS``).  Calls that overlap on one device share the
     scratch and race; order them on one stream."""
-    import ctypes
-
     import torch
 
     from warpir_amd.runtime import check, library
@@ -327,69 +329,67 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
     """
     import torch
 
-    planned = variant is None and workspace is None
-    if planned:
-        done = _gemm_plans.run(0, a, b, out)
-        if done is not None:
-            return done
+    rec = NO_RECORDING
+    if variant is None and workspace is None:
+        done, rec = _gemm_plans.run(0, a, b, out)
+        if done:
+            return rec
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[0]:
         raise ValueError(f"gemm: shapes {tuple(a.shape)} @ {tuple(b.shape)} do not chain")
     m, k = a.shape
     n = b.shape[1]
     if k % 8 or n % 8:
         raise ValueError("gemm: K and N must be multiples of 8 (16-byte rows)")
-    rec = Recording(a, b, out)
-    if out is None:
+    given = out is not None
+    if not given:
         out = rec.alloc(torch.empty(m, n, dtype=torch.bfloat16, device=a.device))
     if variant is None:
         variant, tiled = _gemm_route(m, n, k)
-        short = m <= 128 and splitk_count(m, n, k) >= 4
         if workspace is not None:
             # the caller's choice of split-K there; elsewhere it is not read, and no partials are
             # allocated beside it
-            variant = SPLITK_GEMM_VARIANT if short else tiled
-        if not _splitk_operands_ok(a, b, out):
+            variant = SPLITK_GEMM_VARIANT if _always_split(m, n, k) else tiled
+        if given and tuple(out.shape) != (m, n):
+            # split-K, which short M of long K always took, refuses it; the tiled kernels
+            # drop what does not fit and write zeros past the product
+            variant = SPLITK_GEMM_VARIANT if _always_split(m, n, k) else tiled
+        if variant == SPLITK_GEMM_VARIANT and not _splitk_operands_ok(a, b, out):
             # the split-K entry points take dense operands only; the tiled
             # kernel reads row-strided views through the globals' row stride
             variant = tiled
-        elif tuple(out.shape) != (m, n):
-            # split-K, which short M of long K always took, refuses it; the tiled kernels
-            # drop what does not fit and write zeros past the product
-            variant = SPLITK_GEMM_VARIANT if short else tiled
     if variant == SPLITK_GEMM_VARIANT:
-        splits = splitk_count(m, n, k)
-        if planned and a.is_cuda:
+        if rec:
+            splits = splitk_count(m, n, k)
             workspace = rec.alloc(torch.empty(splits * m * n, dtype=torch.float32, device=a.device))
         gemm_split_k(a, b, out=out, workspace=workspace)
-        if planned and a.is_cuda:
+        if rec:
             _record_split_k(rec, a, b, out, workspace, splits)
             _gemm_plans.add(0, rec, out)
         return out
-    handle = kernels.handle(variant)
-    handle(A=a, B=b, N=k, C_global=out)
-    if planned and m and n and k and a.is_cuda:
-        rec.kernel(handle, A=a, B=b, N=k, C_global=out)
+    rec.kernel(kernels.handle(variant), dict(A=a, B=b, N=k, C_global=out))
+    if rec:
         _gemm_plans.add(0, rec, out)
     return out
+
+
+class _ReduceArgs(ctypes.Structure):   # wir_splitk_reduce
+    _fields_ = [("partials", ctypes.c_void_p), ("out", ctypes.c_void_p), ("n", ctypes.c_longlong),
+                ("split_stride", ctypes.c_longlong), ("splits", ctypes.c_int)]
 
 
 def _record_split_k(rec: Recording, a, b, out, ws, splits: int) -> None:
     """The two launches of ``wir_gemm_splitk``: the slices of A and B along
     the depth of their globals, then the reduction."""
-    import ctypes
-
-    class Reduce(ctypes.Structure):
-        _fields_ = [("partials", ctypes.c_void_p), ("out", ctypes.c_void_p), ("n", ctypes.c_longlong),
-                    ("split_stride", ctypes.c_longlong), ("splits", ctypes.c_int)]
-
     (m, k), n = a.shape, b.shape[1]
     kc = k // splits
-    a4, b4, ws4 = a.view(1, m, splits, kc).transpose(1, 2), b.view(1, splits, kc, n), ws.view(1, splits, m, n)
-    rec.kernel(kernels.handle(SPLITK_GEMM_VARIANT), A=a4, B=b4, N=kc, C_global=ws4,
-               addend={"A": (a, 0), "B": (b, 0), "C_global": (ws, 0)})
-    _, reduce_fn = _splitk_functions(SPLITK_GEMM_VARIANT)
-    rec.raw(reduce_fn, ((m * n // 8 + 255) // 256, 1, 1), (256, 1, 1), Reduce(0, 0, m * n, m * n, splits),
-            [(Reduce.partials.offset, rec.slot(ws), 0), (Reduce.out.offset, rec.slot(out), 0)])
+    args_type = kernels.handle(SPLITK_GEMM_VARIANT).args_type
+    args = args_type(A=GL(0, 1, splits, m, kc, 0, kc, k), B=GL(0, 1, splits, kc, n, 0, kc * n, n), N=kc,
+                     C_global=GL(0, 1, splits, m, n, 0, m * n, n))
+    gemm_fn, reduce_fn = _splitk_functions(SPLITK_GEMM_VARIANT)
+    rec.raw(gemm_fn, (math.ceil(n / 128), math.ceil(m / 128), splits), (256, 1, 1), args,
+            [(getattr(args_type, f).offset, rec.slot(t), 0) for f, t in (("A", a), ("B", b), ("C_global", ws))])
+    rec.raw(reduce_fn, ((m * n // 8 + 255) // 256, 1, 1), (256, 1, 1), _ReduceArgs(0, 0, m * n, m * n, splits),
+            [(_ReduceArgs.partials.offset, rec.slot(ws), 0), (_ReduceArgs.out.offset, rec.slot(out), 0)])
 
 
 def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
@@ -401,10 +401,11 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     import torch
 
     planned = variant is None and type(causal) in (bool, int) and 0 <= causal <= 1   # others are refused below
+    rec = NO_RECORDING
     if planned:
-        done = _forward_plans.run(1 if causal else 0, q, k, v, out, lse)
-        if done is not None:
-            return done
+        done, rec = _forward_plans.run(1 if causal else 0, q, k, v, out, lse)
+        if done:
+            return rec
     bsz, heads, seq, d = q.shape
     hr = _head_ratio("attention_forward", q, k, v)
     if variant is None:
@@ -420,32 +421,31 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
             # 336 blocks, B6 H8 S896: 26.5 -> 27.6 us)
             variant = "mha_d128_w4"
     handle = kernels.handle(variant)
-    kv_tile = next(o for o in _loops(handle.kernel)).tile_size
+    kv_tile = _kv_tile(variant)
     if seq % kv_tile:
         raise ValueError(f"attention_forward: S={seq} must be a multiple of the KV tile {kv_tile}")
-    rec = Recording(q, k, v, out, lse)
+    # (the tiled kernels' grid covers destinations of other shapes: what does not fit is dropped)
+    whole = (out is None or out.shape == q.shape) and (lse is None or lse.shape == (bsz, heads, seq))
     if out is None:
         out = rec.alloc(torch.empty_like(q))
     if lse is None:
         lse = rec.alloc(torch.empty(bsz, heads, seq, dtype=torch.float32, device=q.device))
     args = dict(Q=q, K=k, V=v, N=seq, O=out, L=lse)
-    if (planned and _split_kv_fits(bsz, heads, seq, causal, k, v)
-            and out.shape == q.shape and lse.shape == (bsz, heads, seq)):
-        # (the tiled kernels' grid covers destinations of other shapes: what does not fit is dropped)
-        _attention_split_kv(handle, args, hr, causal, rec)
-        return out, lse
-    if any(v_.name == "HR" for v_ in handle.kernel.inputs):
+    if "HR" in handle.args_type.__dict__:
         args["HR"] = hr
     elif hr > 1:
         raise ValueError(f"attention_forward: variant {variant} takes no grouped-query heads")
-    handle(**args)
-    if planned and q.is_cuda and out.numel() and k.numel():
-        rec.kernel(handle, **args)
+    packing = rec.pack(handle, args)
+    if planned and whole and _split_kv_fits(bsz * heads * (seq // 32), causal, packing[0]):
+        _attention_split_kv(packing, args, (bsz, heads, seq, d), hr, causal, rec)
+        return out, lse
+    rec.kernel(handle, args, packing=packing)
+    if rec:
         _forward_plans.add(1 if causal else 0, rec, out, lse)
     return out, lse
 
 
-def _split_kv_fits(bsz: int, heads: int, seq: int, causal: bool, k, v) -> bool:
+def _split_kv_fits(programs: int, causal: bool, packed) -> bool:
     """Whether the forward goes to the split-key kernel
     (``attn_splitkv.hip``, 32 query rows per program, one program per CU).
     It wins while its programs fit the CUs once, and causal ones, half of them
@@ -454,39 +454,38 @@ def _split_kv_fits(bsz: int, heads: int, seq: int, causal: bool, k, v) -> bool:
     programs S2048 D64 30.0 -> 26.5 and D128 46.5 -> 48.5, causal 29.3 -> 18.5
     and 41.1 -> 31.1; at 1024 B2 H8 S2048 D64 31.8 -> 49.9.  Its lane offsets
     are 32-bit."""
-    return (0 < bsz * heads * (seq // 32) <= (512 if causal else 256)
-            and all(0 <= t.stride(2) < 1 << 23 for t in (k, v)))
+    return (0 < programs <= (512 if causal else 256)
+            and 0 <= packed.K.sr < 1 << 23 and 0 <= packed.V.sr < 1 << 23)
 
 
 _split_kv_kernels: dict = {}
 
 
-def _attention_split_kv(handle, args: dict, hr: int, causal: bool, rec: Recording) -> None:
-    """Launch the split-key forward on the arguments of the tiled kernel
-    *handle*, which validates and packs them, and keep the call's plan."""
-    import ctypes
+class _SplitKvArgs(ctypes.Structure):
+    _fields_ = [("Q", GL), ("K", GL), ("V", GL), ("N", ctypes.c_int), ("HR", ctypes.c_int), ("O", GL), ("L", GL)]
 
+
+_SPLIT_KV_POINTERS = [(f, getattr(_SplitKvArgs, f).offset) for f in "QKVOL"]
+
+
+def _attention_split_kv(packing, args: dict, shape, hr: int, causal: bool, rec) -> None:
+    """Launch the split-key forward on what a tiled kernel's handle made of
+    *args* (validated, packed; *shape* is Q's), and keep the call's plan."""
     import torch
 
-    from warpir_amd.runtime import GL, RawKernel
-
-    class Args(ctypes.Structure):
-        _fields_ = [("Q", GL), ("K", GL), ("V", GL), ("N", ctypes.c_int), ("HR", ctypes.c_int), ("O", GL), ("L", GL)]
-
-    if "HR" in handle.args_type.__dict__:
-        args = {**args, "HR": hr}
-    packed, _cfg, device, _empty = handle.pack(args)
-    name = f"wir_attn_splitkv_d{args['Q'].shape[3]}" + ("_causal" if causal else "")
+    packed, _cfg, device, _empty = packing
+    bsz, heads, seq, d = shape
+    name = f"wir_attn_splitkv_d{d}" + ("_causal" if causal else "")
     kernel = _split_kv_kernels.get(name)
     if kernel is None:
         kernel = _split_kv_kernels.setdefault(name, RawKernel("attn_splitkv.hsaco", name))
-    packed = Args(packed.Q, packed.K, packed.V, args["N"], hr, packed.O, packed.L)
-    bsz, heads, seq, _ = args["Q"].shape
+    packed = _SplitKvArgs(packed.Q, packed.K, packed.V, args["N"], hr, packed.O, packed.L)
     grid, block = (seq // 32, heads, bsz), (256, 1, 1)
     kernel.launch(grid, block, packed, stream=torch.cuda.current_stream(device).cuda_stream)
-    rec.raw(kernel._function, grid, block, packed,
-            [(getattr(Args, f).offset, rec.slot(args[f]), 0) for f in "QKVOL"])
-    _forward_plans.add(1 if causal else 0, rec, args["O"], args["L"])
+    if rec:
+        rec.raw(kernel._function, grid, block, packed,
+                [(offset, rec.slot(args[f]), 0) for f, offset in _SPLIT_KV_POINTERS])
+        _forward_plans.add(1 if causal else 0, rec, args["O"], args["L"])
 
 
 def _head_ratio(fn: str, q, k, v) -> int:
@@ -519,10 +518,11 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     import torch
 
     planned = workspace is None
+    rec = NO_RECORDING
     if planned:
-        done = _backward_plans.run(1 if causal else 0, q, k, v, o, lse, do, dq, dk, dv, dvec)
-        if done is not None:
-            return done
+        done, rec = _backward_plans.run(1 if causal else 0, q, k, v, o, lse, do, dq, dk, dv, dvec)
+        if done:
+            return rec
     if q.dim() != 4 or not (q.shape == o.shape == do.shape):
         raise ValueError("attention_backward: q, o, do must share one [B, H, S, D] shape")
     hr = _head_ratio("attention_backward", q, k, v)
@@ -531,7 +531,8 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
         raise ValueError(f"attention_backward: D must be 64 or 128 and S a multiple of 64 (got D={d}, S={seq})")
     if tuple(lse.shape) != (bsz, heads, seq) or lse.dtype != torch.float32:
         raise ValueError("attention_backward: lse must be fp32 [B, H, S]")
-    rec = Recording(q, k, v, o, lse, do, dq, dk, dv, dvec)
+    whole = (all(g is None or g.shape == q.shape for g in (dq, dk, dv))   # as in the forward
+             and (dvec is None or dvec.shape == lse.shape))
     dq = rec.alloc(torch.empty_like(q)) if dq is None else dq
     dk = rec.alloc(torch.empty_like(k)) if dk is None else dk
     dv = rec.alloc(torch.empty_like(v)) if dv is None else dv
@@ -557,19 +558,17 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     # (handle, arguments, views) of each launch in order
     launches = [(kernels.handle(f"mha_bwd_dq_prep_d{d}{sfx}"), dq_args, None),
                 (kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}"), dkdv_args, views)]
-    if (planned and hr == 1 and _split_bwd_fits(bsz, heads, seq, q, k, v, do)
-            and all(g.shape == q.shape for g in (dq, dk, dv)) and dvec.shape == lse.shape):   # as in the forward
+    if planned and whole and hr == 1 and _split_bwd_fits(bsz, heads, seq, q, k, v, do):
         _attention_bwd_split(launches, causal, rec, dvec)
-        _backward_plans.add(1 if causal else 0, rec, dq, dk, dv)
+        if rec:
+            _backward_plans.add(1 if causal else 0, rec, dq, dk, dv)
         return dq, dk, dv
-    for handle, args, _ in launches:
-        handle(**args)
+    for handle, args, seen in launches:
+        rec.kernel(handle, args, seen)
     reductions = []
     if hr > 1:
         reductions = [(_group_reduce(dk_part, dk, hr), 0, dk), (_group_reduce(dv_part, dv, hr), 4 * numel, dv)]
-    if planned and q.is_cuda and q.numel() and k.numel():
-        for handle, args, seen in launches:
-            rec.kernel(handle, addend=seen, **args)
+    if rec:
         for (grid, args), off, grad in reductions:
             rec.raw(_group_reduce_kernel._function, grid, (256, 1, 1), args,
                     [(type(args).partials.offset, rec.slot(workspace), off), (type(args).out.offset, rec.slot(grad), 0)])
@@ -590,12 +589,10 @@ def _split_bwd_fits(bsz: int, heads: int, seq: int, *loaded) -> bool:
 _split_bwd_kernels: dict = {}
 
 
-def _attention_bwd_split(launches, causal: bool, rec: Recording, dvec) -> None:
+def _attention_bwd_split(launches, causal: bool, rec, dvec) -> None:
     """Launch the split dQ and dK/dV kernels on the arguments of the tiled
     kernels in *launches*, which validate and pack them, and record them."""
     import torch
-
-    from warpir_amd.runtime import RawKernel
 
     stream = torch.cuda.current_stream(dvec.device).cuda_stream
     for part, (handle, args, _) in zip(("dq", "dkdv"), launches):
@@ -604,32 +601,29 @@ def _attention_bwd_split(launches, causal: bool, rec: Recording, dvec) -> None:
         kernel = _split_bwd_kernels.get(name)
         if kernel is None:
             kernel = _split_bwd_kernels.setdefault(name, RawKernel("attn_bwd_split.hsaco", name))
-        packed = handle.pack(args)[0]
+        packed = rec.pack(handle, args)[0]
         grid, block = (seq // 32, heads, bsz), (256, 1, 1)
         kernel.launch(grid, block, packed, stream=stream)
-        rec.raw(kernel._function, grid, block, packed,
-                [(getattr(handle.args_type, f).offset, rec.slot(x), 0) for f, x in args.items()
-                 if isinstance(x, torch.Tensor)])
+        if rec:
+            rec.raw(kernel._function, grid, block, packed,
+                    [(getattr(handle.args_type, f).offset, rec.slot(x), 0) for f, x in args.items()
+                     if isinstance(x, torch.Tensor)])
 
 
 _group_reduce_kernel = None
 
 
+class _GroupReduceArgs(ctypes.Structure):
+    _fields_ = [("partials", ctypes.c_void_p), ("out", ctypes.c_void_p), ("n", ctypes.c_longlong),
+                ("groups", ctypes.c_longlong), ("splits", ctypes.c_int)]
+
+
 def _group_reduce(partials, out, splits: int):
     """``out[g] = bf16(sum_r partials[g * splits + r])`` over the key/value head
     groups of a ``[B, H, S, D]`` fp32 contribution tensor (``splitk_reduce.hip``)."""
-    import ctypes
-
-    from warpir_amd.runtime import RawKernel
-
     global _group_reduce_kernel
     if _group_reduce_kernel is None:
         _group_reduce_kernel = RawKernel("splitk_reduce.hsaco", "wir_group_reduce")
-
-    class Args(ctypes.Structure):
-        _fields_ = [("partials", ctypes.c_void_p), ("out", ctypes.c_void_p), ("n", ctypes.c_longlong),
-                    ("groups", ctypes.c_longlong), ("splits", ctypes.c_int)]
-
     if not out.is_contiguous() or out.dtype.itemsize != 2:
         raise ValueError("attention_backward: dk / dv must be contiguous bf16")
     if out.numel() == 0:
@@ -638,7 +632,7 @@ def _group_reduce(partials, out, splits: int):
     groups = out.numel() // n
     if n % 8 or partials.numel() != groups * splits * n:
         raise ValueError("attention_backward: grouped reduction needs S * D % 8 == 0 and matching shapes")
-    args = Args(partials.data_ptr(), out.data_ptr(), n, groups, splits)
+    args = _GroupReduceArgs(partials.data_ptr(), out.data_ptr(), n, groups, splits)
     grid = ((groups * n // 8 + 255) // 256, 1, 1)
     _group_reduce_kernel.launch(grid, (256, 1, 1), args)
     return grid, args
@@ -659,9 +653,11 @@ def attention_flops(bsz: int, heads: int, seq: int, d: int, causal: bool = False
     return f / 2 if causal else f
 
 
-def _loops(kernel):
+@functools.lru_cache(maxsize=None)
+def _kv_tile(variant: str) -> int:
     from warpir_amd.ir.ops import ForOp
-    return (op for op in kernel.body if isinstance(op, ForOp))
+
+    return next(op for op in kernels.handle(variant).kernel.body if isinstance(op, ForOp)).tile_size
 
 
 __all__ = ["gemm", "gemm_split_k", "splitk_count", "gemm_variant", "attention_forward", "attention_backward",

@@ -9,12 +9,15 @@
 // function, grid and argument bytes with the places of the tensor pointers.
 // A later call with the same signature allocates, fills the pointers in and
 // launches.  Nothing is kept by a tensor's address or identity, and a table
-// holds at most MAX_PLANS plans (it starts over when full).
+// holds at most MAX_PLANS plans (a new one then takes the place of another,
+// drawn at random: a program that goes round more signatures than that still
+// finds part of them, where dropping the oldest or all would find none).
 //
-// run() returns None for every call that it does not know or must not take
-// (tensor subclasses, functorch or Python-dispatch wrappers, active torch
-// function / dispatch modes, empty or not 16-byte aligned tensors), and the
-// Python path then does, with its own checks and errors.  The interpreter
+// run() returns False for every call that it does not know and None for those
+// it must not take (tensor subclasses, functorch or Python-dispatch wrappers,
+// active torch function / dispatch modes, empty or not 16-byte aligned
+// tensors); the Python path then does, with its own checks and errors, and
+// leaves a plan after False only.  The interpreter
 // lock guards the tables; it is released around the launches only.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -67,7 +70,29 @@ struct Plan {
   std::vector<int> results;   // slots
 };
 
-typedef std::unordered_map<std::string, std::shared_ptr<Plan>> Table;
+struct Table {
+  std::unordered_map<std::string, std::shared_ptr<Plan>> plans;
+  std::vector<const std::string*> keys;   // of every plan (a map's keys stay where they are)
+  uint32_t draw = 0x9e3779b9u;            // xorshift state
+
+  void keep(const std::string& key, std::shared_ptr<Plan> plan) {
+    auto found = plans.find(key);
+    if (found != plans.end()) {
+      found->second = std::move(plan);
+      return;
+    }
+    auto it = plans.emplace(key, std::move(plan)).first;
+    if (keys.size() < MAX_PLANS) {
+      keys.push_back(&it->first);
+      return;
+    }
+    draw ^= draw << 13, draw ^= draw >> 17, draw ^= draw << 5;
+    const std::string*& slot = keys[draw % MAX_PLANS];
+    const std::string old = *slot;
+    slot = &it->first;
+    plans.erase(old);
+  }
+};
 
 const char* kTableName = "warpir_amd.plans.Table";
 
@@ -87,17 +112,13 @@ bool plain(const at::Tensor& t) {
 
 // The signature of `flags` and the tensors (None allowed) args[0..n), whose
 // tensors go to `slots`; false when the call is not one for a plan.
-bool signature(PyObject* flags, PyObject* const* args, Py_ssize_t n, std::string& key, const at::Tensor** slots,
+bool signature(long long flags, PyObject* const* args, Py_ssize_t n, std::string& key, const at::Tensor** slots,
                int* device) {
   if (n > MAX_SLOTS || c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled())
     return false;
   long long buf[2 + MAX_SLOTS * 18];
   int w = 0;
-  buf[w++] = PyLong_AsLongLong(flags);
-  if (PyErr_Occurred()) {
-    PyErr_Clear();
-    return false;
-  }
+  buf[w++] = flags;
   *device = -1;
   for (Py_ssize_t i = 0; i < n; ++i) {
     slots[i] = nullptr;
@@ -122,8 +143,25 @@ bool signature(PyObject* flags, PyObject* const* args, Py_ssize_t n, std::string
   return true;
 }
 
+bool flags_of(PyObject* o, long long* flags) {
+  *flags = PyLong_AsLongLong(o);
+  if (!PyErr_Occurred()) return true;
+  PyErr_Clear();
+  return false;
+}
+
+// Whether no tensor is given twice: the launches of a call that gives one
+// twice do not tell which argument a pointer came from.
+bool distinct(PyObject* const* args, Py_ssize_t n) {
+  for (Py_ssize_t i = 0; i < n; ++i)
+    for (Py_ssize_t j = i + 1; j < n; ++j)
+      if (args[i] == args[j] && args[i] != Py_None) return false;
+  return true;
+}
+
 // run(table, flags, *tensors) -> the plan's result tensors (one, or a tuple),
-// an int error code of a failed launch, or None.
+// an int error code of a failed launch, False where the call has no plan yet
+// and can leave one, or None where it can not.
 PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (nargs < 3 || !g_launch) Py_RETURN_NONE;
@@ -133,9 +171,13 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const at::Tensor* slots[MAX_SLOTS];
   std::string key;
   int device = -1;
-  if (!signature(args[1], args + 2, n, key, slots, &device)) Py_RETURN_NONE;
-  auto it = table->find(key);
-  if (it == table->end()) Py_RETURN_NONE;
+  long long flags;
+  if (!flags_of(args[1], &flags) || !signature(flags, args + 2, n, key, slots, &device)) Py_RETURN_NONE;
+  auto it = table->plans.find(key);
+  if (it == table->plans.end()) {
+    if (distinct(args + 2, n)) Py_RETURN_FALSE;
+    Py_RETURN_NONE;
+  }
   const std::shared_ptr<Plan> plan = it->second;   // stays alive if another thread drops it from the table
 
   std::vector<at::Tensor> made;
@@ -213,7 +255,10 @@ PyObject* add(PyObject*, PyObject* args) {
   std::string key;
   int device = -1;
   if (n + made > MAX_SLOTS || n < 1) Py_RETURN_FALSE;
-  if (!signature(flags, &PyTuple_GET_ITEM(inputs, 0), n, key, slots, &device)) Py_RETURN_FALSE;
+  long long bits;
+  PyObject* const* given = &PyTuple_GET_ITEM(inputs, 0);
+  if (!flags_of(flags, &bits) || !distinct(given, n) || !signature(bits, given, n, key, slots, &device))
+    Py_RETURN_FALSE;
   auto plan = std::make_shared<Plan>();
   for (Py_ssize_t i = 0; i < made; ++i) {
     PyObject* o = PyList_GET_ITEM(allocs, i);
@@ -251,8 +296,7 @@ PyObject* add(PyObject*, PyObject* args) {
     plan->results.push_back((int)s);
   }
   if (plan->results.empty()) Py_RETURN_FALSE;
-  if (table->size() >= MAX_PLANS) table->clear();
-  (*table)[key] = std::move(plan);
+  table->keep(key, std::move(plan));
   Py_RETURN_TRUE;
   END_HANDLE_TH_ERRORS
 }
@@ -260,7 +304,7 @@ PyObject* add(PyObject*, PyObject* args) {
 // size(table): the number of plans held.
 PyObject* size(PyObject*, PyObject* capsule) {
   Table* table = table_of(capsule);
-  return table ? PyLong_FromSize_t(table->size()) : nullptr;
+  return table ? PyLong_FromSize_t(table->plans.size()) : nullptr;
 }
 
 PyObject* new_table(PyObject*, PyObject*) { return PyCapsule_New(new Table, kTableName, free_table); }

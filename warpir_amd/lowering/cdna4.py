@@ -236,6 +236,7 @@ class CDNA4Lowerer:
 
     def __init__(self, target: Optional[CDNA4Target] = None):
         self.target = target or CDNA4Target()
+        self._grid_axes: Optional[tuple] = None   # launch_config's, of the kernel it was last asked for
         self._reset()
 
     # ------------------------------------------------------------------
@@ -324,17 +325,21 @@ class CDNA4Lowerer:
         """Grid / block for concrete output shapes (``tensors``: name -> shape)."""
         if self.kernel is not kernel:
             self.lower(kernel)
+        if self._grid_axes is None or self._grid_axes[0] is not kernel:
+            axes = []   # (global, coordinate, grid axis, tile extent) of every store
+            for op in _walk(kernel.body):
+                if isinstance(op, TMAStoreOp):
+                    sub = op.dest.type.sub_tile_type
+                    axes += [(op.dest.name, pos, BUILTINS.index(c.name), unit)
+                             for pos, (c, unit) in enumerate(zip(op.coords, (1, 1, sub.rows, sub.cols)))
+                             if isinstance(c, Value) and c.name in BUILTINS]
+            self._grid_axes = (kernel, axes)
         grid = [1, 1, 1]
-        for op in _walk(kernel.body):
-            if not isinstance(op, TMAStoreOp):
-                continue
-            shape = _as4d(tensors[op.dest.name])
-            sub = op.dest.type.sub_tile_type
-            units = (1, 1, sub.rows, sub.cols)
-            for pos, c in enumerate(op.coords):
-                if isinstance(c, Value) and c.name in BUILTINS:
-                    axis = BUILTINS.index(c.name)
-                    grid[axis] = max(grid[axis], _ceil_div(shape[pos], units[pos]))
+        shapes = {}
+        for name, pos, axis, unit in self._grid_axes[1]:
+            if name not in shapes:
+                shapes[name] = _as4d(tensors[name])
+            grid[axis] = max(grid[axis], _ceil_div(shapes[name][pos], unit))
         if self.target.persistent:
             total = grid[0] * grid[1] * grid[2]
             grid = [max(1, min(total, self.target.persistent)), 1, 1]

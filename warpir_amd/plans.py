@@ -45,37 +45,65 @@ class Recording:
         self.inputs = inputs
         self.allocs = []
         self.launches = []
+        self._slots = {id(t): i for i, t in enumerate(inputs)}
 
     def alloc(self, t):
         """Note that the call allocated *t*."""
+        self._slots[id(t)] = len(self.inputs) + len(self.allocs)
         self.allocs.append(t)
         return t
 
     def slot(self, t) -> int:
-        for i, x in enumerate(self.inputs):
-            if x is t:
-                return i
-        return len(self.inputs) + next(i for i, x in enumerate(self.allocs) if x is t)
+        return self._slots[id(t)]   # (inputs and allocations outlive the recording)
 
-    def kernel(self, handle, addend=None, **args) -> None:
-        """A launch of a ``KernelHandle``; ``addend`` maps an argument that is
-        a view to (the tensor it views, its offset in bytes)."""
+    def pack(self, handle, args):
+        """*args* packed for a ``KernelHandle``, past its cache: the next call
+        with this signature takes the plan."""
+        return handle.pack(args)
+
+    def kernel(self, handle, args, addend=None, packing=None) -> None:
+        """Launch a ``KernelHandle`` on *args* (packed as *packing*) and note
+        it; ``addend`` maps an argument that is a view to (the tensor it
+        views, its offset in bytes)."""
         import torch
 
-        packed, cfg, _device, empty = handle.pack(args)
-        if empty or not all(cfg.grid):
+        if packing is None:
+            packing = self.pack(handle, args)
+        packed, cfg = packing[:2]
+        if not handle.launch(packing):
             raise ValueError("an empty launch has no plan")
-        handle.load()
         pointers = []
         for name, x in args.items():
             if isinstance(x, torch.Tensor):
-                base, off = (addend or {}).get(name, (x, 0))
+                base, off = addend[name] if addend and name in addend else (x, 0)
                 pointers.append((getattr(handle.args_type, name).offset, self.slot(base), off))
         self.raw(handle._function, cfg.grid, cfg.block, packed, pointers, cfg.dyn_lds)
 
     def raw(self, function, grid, block, args, pointers, dyn_lds: int = 0) -> None:
-        """A launch of a loaded function with a ctypes argument structure."""
+        """Note a launch of a loaded function with a ctypes argument structure."""
         self.launches.append((function.value, tuple(grid), tuple(block), dyn_lds, bytes(args), pointers))
+
+
+class _NoRecording:
+    """In the place of the recording of a call that can have no plan."""
+
+    def alloc(self, t):
+        return t
+
+    def pack(self, handle, args):
+        return handle.packed(args)
+
+    def kernel(self, handle, args, addend=None, packing=None) -> None:
+        if packing is None:
+            handle(**args)
+        else:
+            handle.launch(packing)
+
+    def __bool__(self) -> bool:
+        return False
+
+
+NO_RECORDING = _NoRecording()
 
 
 class Plans:
@@ -86,30 +114,34 @@ class Plans:
         self._table = None
 
     def run(self, flags: int, *tensors):
-        """The call's results by its plan, or None where it has none."""
+        """(whether the call ran by its plan, its results; or the recording of
+        a call that has none: ``NO_RECORDING`` where none can be kept, so that
+        nothing is packed for it in vain).  us, without plans / recording in
+        vain / now: gemm under ``torch.set_default_device`` 28 / 68 / 28,
+        the tiled backward 123 / 289 / 109."""
         table = self._table
         if table is None:
-            return None
-        r = _native.run(table, flags, *tensors)
-        if type(r) is int:
-            from warpir_amd.runtime import check
-
-            check(r, self.what)
-        return r
-
-    def add(self, flags: int, rec: Recording, *results) -> None:
-        """Keep the plan of a call that has just run.  A call that passed one
-        tensor twice gives none: its launches do not tell which argument a
-        pointer came from."""
-        given = [id(t) for t in rec.inputs if t is not None]
-        if len(set(given)) != len(given):
-            return
-        if self._table is None:
+            if _native is None and not getattr(tensors[0], "is_cuda", False):
+                return False, NO_RECORDING
             mod = native()
             with _lock:
                 if self._table is None:
                     self._table = mod.table()
+                table = self._table
+        r = _native.run(table, flags, *tensors)
+        if r is None:
+            return False, NO_RECORDING
+        if r is False:
+            return False, Recording(*tensors)
+        if type(r) is int:
+            from warpir_amd.runtime import check
+
+            check(r, self.what)
+        return True, r
+
+    def add(self, flags: int, rec: Recording, *results) -> None:
+        """Keep the plan of a call that has just run."""
         _native.add(self._table, flags, rec.inputs, rec.allocs, rec.launches, [rec.slot(t) for t in results])
 
 
-__all__ = ["Plans", "Recording", "native"]
+__all__ = ["Plans", "Recording", "NO_RECORDING", "native"]

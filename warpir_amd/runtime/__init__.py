@@ -369,9 +369,8 @@ class KernelHandle:
                 return None
         return tuple(sig) if len(args) == len(sig) else None
 
-    def __call__(self, stream=None, **args) -> None:
-        import torch
-
+    def packed(self, args: Dict[str, object]):
+        """``pack(args)``, kept for the next call with the same tensors."""
         key = self._signature(args)
         hit = self._pack_cache.get(key) if key is not None else None
         if hit is None:
@@ -380,10 +379,17 @@ class KernelHandle:
                 if len(self._pack_cache) >= 64:
                     self._pack_cache.clear()
                 self._pack_cache[key] = hit
-        packed, cfg, device, empty = hit
+        return hit
+
+    def launch(self, packing, stream=None) -> bool:
+        """Launch on what ``pack`` or ``packed`` returned; False where there is
+        nothing to launch."""
+        import torch
+
+        packed, cfg, device, empty = packing
         gx, gy, gz = cfg.grid
         if empty or not (gx and gy and gz):
-            return   # an empty problem: no output element to write, or no workgroup
+            return False   # an empty problem: no output element to write, or no workgroup
         self.load()
         if stream is None:
             stream = torch.cuda.current_stream(device).cuda_stream
@@ -393,6 +399,10 @@ class KernelHandle:
         check(library().wir_launch(self._function, gx, gy, gz, bx, by, bz, cfg.dyn_lds,
                                    ctypes.c_void_p(stream), ctypes.byref(packed), ctypes.sizeof(packed)),
               f"wir_launch({self.kernel.name})")
+        return True
+
+    def __call__(self, stream=None, **args) -> None:
+        self.launch(self.packed(args), stream)
 
     def __del__(self):
         if self._module is not None and _lib is not None:
