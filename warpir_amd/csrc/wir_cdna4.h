@@ -1929,14 +1929,9 @@ __device__ __forceinline__ int remap_xcd(int hw_id, int total) {
 //   dK/dV    B16 H16 S1024 D128      266 / 227 / 215 / 216 / 218
 //   forward  B8 H32 S8192 D64       2436 / 2403 / 2370 / 2416 / 3162
 // (all heads by length lose the L2's hold on K and V where they are many and long).
-// The key-major kernel (!REVERSE) streams Q and dO of one query head, which no
-// other head shares, and its blocks of one head start at different rows: past
-// 16 blocks a head the order costs it more in L2 misses than its tail saves
-// (in a training step, us: S4096 2952 -> 2979, S5504 1980 -> 2303, against
-// S2048 205 -> 168, S1024 257 -> 225), so longer heads run in turn.
 template <bool REVERSE, int TAIL>
 __device__ __forceinline__ void longest_first(int hw, int nx, int heads, int& x, int& head) {
-  const int tail = !REVERSE && nx > 16 ? 0 : min(heads, max(8, TAIL / nx & ~7)), lead = heads - tail;
+  const int tail = min(heads, max(8, TAIL / nx & ~7)), lead = heads - tail;
   if (hw < lead * nx) {
     const int id = remap_xcd(hw, lead * nx);
     x = id % nx;
