@@ -44,7 +44,10 @@ struct Scale {
   static constexpr float s = (float)inv_sqrt, c = (float)(1.4426950408889634 * inv_sqrt);
 };
 
-// Program -> (block of 32 rows, head, batch); causal launches end on the short blocks.
+// Program -> (block of 32 rows, head, batch); causal launches end on the short
+// blocks (the LDS holds one workgroup per CU, so the order sets the tail: dK/dV,
+// heads in turn -> this order, B1 H4 S4096 D64 52.8 -> 40.2 us, H20 S768 D64 19.1 ->
+// 16.0, H12 S1024 D128 27.2 -> 24.3, H8 S2048 D64 25.1 -> 25.0).
 template <bool CAUSAL, bool REVERSE>
 __device__ __forceinline__ void program(int& x, int& h, int& b) {
   const int nx = gridDim.x, ny = gridDim.y, heads = ny * gridDim.z;

@@ -1923,12 +1923,18 @@ __device__ __forceinline__ int remap_xcd(int hw_id, int total) {
 // that share K and V).
 //
 // TAIL = 2048 is two to four blocks per slot (256 CUs x 2 or 3 workgroups).
-// us, every head in turn / 1024 / 2048 / 4096 / all heads by length:
-//   forward  B1 H32/8 S4096 D128     172 / 139 / 139 / 138 / 142
-//   forward  B16 H16 S4096 D128     1298 / 1209 / 1212 / 1255 / 1385
-//   dK/dV    B16 H16 S1024 D128      266 / 227 / 215 / 216 / 218
-//   forward  B8 H32 S8192 D64       2436 / 2403 / 2370 / 2416 / 3162
-// (all heads by length lose the L2's hold on K and V where they are many and long).
+// us, every head in turn / 1024 / 2048 / 4096 (launches of the four in turn, so
+// that the clocks' drift of several per cent between runs falls on all alike):
+//   forward  B1 H32/8 S4096 D128     176 / 141 / 142 / 142
+//   forward  B16 H16 S4096 D128     1170 / 1134 / 1121 / 1173
+//   forward  B8 H32 S8192 D64       2314 / 2302 / 2268 / 2252
+//   dQ       B16 H16 S4096 D128     1653 / 1574 / 1560 / 1547
+//   dK/dV    B16 H16 S1024 D128      257 / 227 / 215 / 216
+//   dK/dV    B4 H16 S2560 D128       288 / 256 / 253 / 253
+//   dK/dV    B16 H16 S4096 D128     2530 / 2468 / 2438 / 2419
+//   dK/dV    B15 H8/4 S5504 D128    2022 / 1993 / 1976 / 1959
+// (all heads by length, with none before them, lose the L2's hold on K and V
+// where they are many and long: forward B8 H32 S8192 D64 3162 against 2370.)
 template <bool REVERSE, int TAIL>
 __device__ __forceinline__ void longest_first(int hw, int nx, int heads, int& x, int& head) {
   const int tail = min(heads, max(8, TAIL / nx & ~7)), lead = heads - tail;
