@@ -75,3 +75,14 @@ def test_operands_that_split_k_does_not_take_get_the_fastest_tile(m, n, k):
     assert route == api.SPLITK_GEMM_VARIANT
     est = {v: api._tiled_estimate(c, m, n, k) for v, c in api._TILE_COST.items()}
     assert est[fallback] == min(est.values())
+
+
+@pytest.mark.parametrize("m,n,k,variant", [
+    (64, 8192, 104, "gemm_64_k64"), (128, 8192, 512, "gemm_64_k64"), (256, 8192, 512, "gemm_128x64_k64"), (2048, 2048, 2048, "gemm_128_k64_s3"),
+    (64, 8192, 8192, "gemm_128_splitk_k64_b7")])
+def test_routes_of_products_that_the_call_accepts(taken, m, n, k, variant):
+    """The call takes the kernel of ``gemm_variant`` with its own K."""
+    want = api.gemm_variant(m, n, k)
+    assert variant in (None, want)
+    api.gemm(_bf16(m, k), _bf16(k, n))
+    assert taken == ["split-K" if want == api.SPLITK_GEMM_VARIANT else want]

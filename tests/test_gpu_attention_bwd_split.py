@@ -69,3 +69,37 @@ def test_split_backward_is_left_at_its_limits(gpu, taken):
         o, lse = api.attention_forward(q, k, k.clone())
         api.attention_backward(q, k, k.clone(), o, lse, q.clone())
         assert len(taken) == want
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+@pytest.mark.parametrize("where", ["k", "v", "q", "do"])
+def test_split_backward_special_values(gpu, taken, monkeypatch, where, bad, d, causal):
+    """A row of NaN or infinities spoils every gradient that depends on it, and
+    no element that the tiled kernels keep finite."""
+    announce(f"split backward {where} {bad} D{d} causal={causal}")
+    host = dict(zip(("q", "k", "v", "do"), (seeded_normal((1, 2, 256, d), s) for s in range(4))))
+    host[where][0, 1, 200] = bad
+    q, k, v, do = (host[x].cuda() for x in ("q", "k", "v", "do"))
+    o, lse = api.attention_forward(q, k, v, causal=causal)
+    got = api.attention_backward(q, k, v, o, lse, do, causal=causal)
+    assert taken
+    monkeypatch.setattr(api, "_split_bwd_fits", lambda *a: False)
+    monkeypatch.setattr(api, "_backward_plans", api.Plans("attention_backward"))
+    tiled = api.attention_backward(q, k, v, o, lse, do, causal=causal)
+    assert len(taken) == 1
+    exact = attention_bwd_ref(*(host[x] for x in ("q", "k", "v", "do")), causal=causal)
+    # the query rows whose O, LSE or dP see the bad row, and the keys that those rows see
+    i = torch.arange(256)
+    rows = (i >= 200 if causal else i >= 0) if where in ("k", "v") else i == 200
+    keys = i <= (255 if where in ("k", "v") else 200) if causal else i >= 0
+    spoiled = rows, keys, keys & (where != "v")
+    for g, t, e, bad_rows in zip(got, tiled, exact, spoiled):
+        g, t = g.cpu().float(), t.cpu().float()
+        assert not bool(g[0, 1, bad_rows].isfinite().any())
+        assert int((t.isfinite() & ~g.isfinite()).sum()) == 0
+        assert bool(g[0, 0].isfinite().all())   # the other head
+        # (where the fp32 reference is finite: its 0 * NaN of masked scores is NaN, theirs often not formed)
+        both = g.isfinite() & e.isfinite()
+        assert rel_err(g[both], e[both]) <= 1e-2

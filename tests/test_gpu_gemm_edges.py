@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle.torch_ref import gemm_ref, rel_err, seeded_normal
-from warpir_amd import kernels
+from warpir_amd import api, kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +83,19 @@ def test_small_tiles_match_the_256_tile_bit_for_bit(gpu, variant, m, n, k):
     kernels.handle(variant)(A=a, B=b, N=k, C_global=c)
     kernels.handle("gemm_256_k64")(A=a, B=b, N=k, C_global=ref)
     assert torch.equal(c, ref)
+
+
+@pytest.mark.parametrize("m,n,k", [(200, 1024, 8192), (333, 264, 4096), (16, 8192, 6336)])
+def test_split_k_by_estimate(gpu, monkeypatch, m, n, k):
+    """Products that no fixed rule sends to split-K (M > 128, fewer than four
+    slices), on the first call and by its plan."""
+    assert api.gemm_variant(m, n, k) == api.SPLITK_GEMM_VARIANT
+    split, real = [], api.gemm_split_k
+    monkeypatch.setattr(api, "gemm_split_k", lambda *a, **kw: split.append(1) or real(*a, **kw))
+    monkeypatch.setattr(api, "_gemm_plans", api.Plans("gemm"))
+    for seed in (0, 2):
+        a, b = seeded_normal((m, k), seed), seeded_normal((k, n), seed + 1)
+        big, c = _inside(torch.zeros(m, n, dtype=torch.bfloat16, device="cuda"), 8, 0, -7.0)   # rows after the last
+        api.gemm(a.cuda(), b.cuda(), out=c)
+        assert rel_err(c.cpu(), gemm_ref(a, b)) <= TOL and bool((big[m:] == -7.0).all())
+    assert len(split) == 1
