@@ -20,9 +20,10 @@ from warpir_amd.plans import NO_RECORDING, Plans, Recording
 from warpir_amd.runtime import GL, RawKernel
 
 # Plans of the calls below, by flags: gemm 0; attention_forward and
-# attention_backward the causal bit.  A stream of calls, before -> after: gemm
-# 256^3 10.7 -> 4.4 us and attention_forward B1 H8 S512 D64 16.0 -> 10.1 us, now
-# the kernels' own time and the gap between launches.
+# attention_backward the causal bit.  A stream of calls, by the Python path -> by
+# its plan: gemm 256^3 10.7 -> 4.8 us (the kernel's 3.8-4.2 and the gap between
+# launches); attention_forward B1 H8 S512 D64 16.0 -> 10.1 us on the tiled kernel
+# and 5.9 on the split-key one, the kernels' own time.
 _gemm_plans = Plans("gemm")
 _forward_plans = Plans("attention_forward")
 _backward_plans = Plans("attention_backward")

@@ -15,11 +15,10 @@
 namespace {
 
 using wir::bf16;
-using wir::bf16x4;
 using wir::bf16x8;
 using wir::f32x4;
-typedef __attribute__((address_space(3))) float lds_float;
-typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+using wir::lds_f32x4;
+using wir::lds_float;
 
 struct dq_args {   // mha_bwd_dq_prep_*
   wir::gl<bf16> Q, K, V, dO, O;
@@ -36,51 +35,13 @@ struct dkdv_args {   // mha_bwd_dkdv_*
   wir::gl<bf16> dK, dV;
 };
 
-constexpr int WAVES = 4, ROWS = 32;
+constexpr int WAVES = wir::SPLIT_WAVES, ROWS = wir::SPLIT_ROWS;
 
 template <int D>
 struct Scale {
   static constexpr double inv_sqrt = D == 64 ? 0.125 : 0.08838834764831845;
   static constexpr float s = (float)inv_sqrt, c = (float)(1.4426950408889634 * inv_sqrt);
 };
-
-// Program -> (block of 32 rows, head, batch); causal launches end on the short
-// blocks (the LDS holds one workgroup per CU, so the order sets the tail: dK/dV,
-// heads in turn -> this order, B1 H4 S4096 D64 52.8 -> 40.2 us, H20 S768 D64 19.1 ->
-// 16.0, H12 S1024 D128 27.2 -> 24.3, H8 S2048 D64 25.1 -> 25.0).
-template <bool CAUSAL, bool REVERSE>
-__device__ __forceinline__ void program(int& x, int& h, int& b) {
-  const int nx = gridDim.x, ny = gridDim.y, heads = ny * gridDim.z;
-  const int hw = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
-  int head;
-  if (CAUSAL) {
-    wir::longest_first<REVERSE, 2048>(hw, nx, heads, x, head);
-  } else {
-    const int id = wir::remap_xcd(hw, nx * heads);
-    x = id % nx;
-    head = id / nx;
-  }
-  h = head % ny;
-  b = head / ny;
-}
-
-// Floats per row of a partial result: 16 rows land in 16 different 16-byte bank slots.
-template <int D>
-constexpr int pitch = D + 4;
-
-template <int D>
-__device__ __forceinline__ void put_partial(lds_float* part, const wir::RTile<32, 32, D>& t, int wave) {
-  const int lane = wir::lane_id(), lr = lane % 32, lh = lane / 32;
-#pragma unroll
-  for (int cb = 0; cb < D / 32; ++cb)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      f32x4 v;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = t.f[cb][0][4 * g + j];
-      *(lds_f32x4*)(part + (wave * ROWS + lr) * pitch<D> + cb * 32 + wir::ccol<32>(4 * g, lh)) = v;
-    }
-}
 
 // bf16 of `scale` times the waves' sum, rows row0.. of one head.
 template <int D>
@@ -96,7 +57,7 @@ __device__ __forceinline__ void store_sum(const lds_float* part, const wir::gl<b
     for (int j = 0; j < 8; ++j) acc[j] = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      const lds_float* p = part + (w * ROWS + row) * pitch<D> + ch * 8;
+      const lds_float* p = part + (w * ROWS + row) * wir::split_pitch<D> + ch * 8;
       const f32x4 lo = *(const lds_f32x4*)p, hi = *(const lds_f32x4*)(p + 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -126,10 +87,10 @@ __device__ __forceinline__ void dq_split(const dq_args& args) {
   typedef wir::STile<KT, D, wir::ROWREAD> TV;
   constexpr int STEP = wir::Loader<TK, 1>::INSTR_PER_WAVE + wir::Loader<TV, 1>::INSTR_PER_WAVE;
   constexpr int SLOT = TK::BYTES + TV::BYTES;
-  static_assert(STEP < 64 && ROWS * pitch<D> * 4 <= 2 * SLOT, "the merge reuses the tiles' LDS");
+  static_assert(STEP < 64 && ROWS * wir::split_pitch<D> * 4 <= 2 * SLOT, "the merge reuses the tiles' LDS");
   __shared__ __attribute__((aligned(1024))) char smem[WAVES * 2 * SLOT];
   int x, h, b;
-  program<CAUSAL, true>(x, h, b);
+  wir::split_program<CAUSAL, true>(x, h, b);
   const int row0 = x * ROWS, wave = wir::wave_id();
   const int tiles = ((CAUSAL ? min(args.N, row0 + ROWS) : args.N) + KT - 1) / KT;
 
@@ -179,7 +140,7 @@ __device__ __forceinline__ void dq_split(const dq_args& args) {
   }
   wir::wait_vm_barrier<0>();
   lds_float* part = (lds_float*)wir::lds(smem);
-  put_partial<D>(part, acc, wave);
+  wir::put_partial<D>(part, acc, wave);
   wir::barrier();
   store_sum<D>(part, args.dQ, b, h, row0, Scale<D>::s);
 }
@@ -191,11 +152,11 @@ __device__ __forceinline__ void dkdv_split(const dkdv_args& args) {
   typedef wir::VecLoader<QT, 1> LoadVec;
   constexpr int STEP = 2 * Load::INSTR_PER_WAVE + 2;
   constexpr int VEC = 2 * T::BYTES, SLOT = VEC + 512;   // Q, dO, then 256 bytes each for the LSE and Dv
-  constexpr int PART = WAVES * ROWS * pitch<D>;
+  constexpr int PART = WAVES * ROWS * wir::split_pitch<D>;
   static_assert(STEP < 64 && QT * 4 <= 256 && 2 * PART * 4 <= WAVES * 2 * SLOT, "the merge reuses the tiles' LDS");
   __shared__ __attribute__((aligned(1024))) char smem[WAVES * 2 * SLOT];
   int x, h, b;
-  program<CAUSAL, false>(x, h, b);
+  wir::split_program<CAUSAL, false>(x, h, b);
   const int row0 = x * ROWS, wave = wir::wave_id();
   const int first = (CAUSAL ? row0 / QT : 0) + wave, tiles = args.N / QT;
 
@@ -245,8 +206,8 @@ __device__ __forceinline__ void dkdv_split(const dkdv_args& args) {
   }
   wir::wait_vm_barrier<0>();
   lds_float* part = (lds_float*)wir::lds(smem);
-  put_partial<D>(part, dk, wave);
-  put_partial<D>(part + PART, dv, wave);
+  wir::put_partial<D>(part, dk, wave);
+  wir::put_partial<D>(part + PART, dv, wave);
   wir::barrier();
   store_sum<D>(part, args.dK, b, h, row0, Scale<D>::s);
   store_sum<D>(part + PART, args.dV, b, h, row0, 1.0f);
@@ -254,16 +215,11 @@ __device__ __forceinline__ void dkdv_split(const dkdv_args& args) {
 
 }  // namespace
 
-#define WIR_KERNEL(NAME, ARGS, CALL)                                                                           \
-  extern "C" __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1))) \
-  NAME(const ARGS args) {                                                                                      \
-    CALL(args);                                                                                                \
-  }
-WIR_KERNEL(wir_attn_dq_split_d64, dq_args, (dq_split<64, 64, false>))
-WIR_KERNEL(wir_attn_dq_split_d64_causal, dq_args, (dq_split<64, 64, true>))
-WIR_KERNEL(wir_attn_dq_split_d128, dq_args, (dq_split<128, 32, false>))
-WIR_KERNEL(wir_attn_dq_split_d128_causal, dq_args, (dq_split<128, 32, true>))
-WIR_KERNEL(wir_attn_dkdv_split_d64, dkdv_args, (dkdv_split<64, 64, false>))
-WIR_KERNEL(wir_attn_dkdv_split_d64_causal, dkdv_args, (dkdv_split<64, 64, true>))
-WIR_KERNEL(wir_attn_dkdv_split_d128, dkdv_args, (dkdv_split<128, 32, false>))
-WIR_KERNEL(wir_attn_dkdv_split_d128_causal, dkdv_args, (dkdv_split<128, 32, true>))
+WIR_SPLIT_KERNEL(wir_attn_dq_split_d64, dq_args, (dq_split<64, 64, false>))
+WIR_SPLIT_KERNEL(wir_attn_dq_split_d64_causal, dq_args, (dq_split<64, 64, true>))
+WIR_SPLIT_KERNEL(wir_attn_dq_split_d128, dq_args, (dq_split<128, 32, false>))
+WIR_SPLIT_KERNEL(wir_attn_dq_split_d128_causal, dq_args, (dq_split<128, 32, true>))
+WIR_SPLIT_KERNEL(wir_attn_dkdv_split_d64, dkdv_args, (dkdv_split<64, 64, false>))
+WIR_SPLIT_KERNEL(wir_attn_dkdv_split_d64_causal, dkdv_args, (dkdv_split<64, 64, true>))
+WIR_SPLIT_KERNEL(wir_attn_dkdv_split_d128, dkdv_args, (dkdv_split<128, 32, false>))
+WIR_SPLIT_KERNEL(wir_attn_dkdv_split_d128_causal, dkdv_args, (dkdv_split<128, 32, true>))

@@ -29,6 +29,8 @@ using wir::bf16;
 using wir::bf16x4;
 using wir::bf16x8;
 using wir::f32x4;
+using wir::lds_f32x4;
+using wir::lds_float;
 
 // Arguments: the grouped-query forward's globals (HR = 1 for plain heads).
 struct splitkv_args {
@@ -39,7 +41,7 @@ struct splitkv_args {
   wir::gl<float> L;
 };
 
-constexpr int WAVES = 4, ROWS = 32;
+constexpr int WAVES = wir::SPLIT_WAVES, ROWS = wir::SPLIT_ROWS;
 constexpr float kLn2 = 0.6931471805599453f;
 
 // Wait until at most `n` of this wave's DMAs are in flight (n = 3, 2, 1 or 0
@@ -102,22 +104,14 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
   typedef wir::Loader<TK, 1> LoadK;
   typedef wir::Loader<TV, 1> LoadV;
   constexpr int STEP = LoadK::INSTR_PER_WAVE, SLOT = TK::BYTES + TV::BYTES;
-  constexpr int PITCH = D + 4;   // floats per row of a partial O: 16 rows land in 16 different 16-byte bank slots
+  constexpr int PITCH = wir::split_pitch<D>;
   static_assert(LoadV::INSTR_PER_WAVE == STEP && 3 * STEP < 64, "vmcnt range");
   static_assert(WAVES * (ROWS * PITCH + 2 * ROWS) * 4 <= WAVES * 2 * SLOT, "the merge reuses the tiles' LDS");
   __shared__ __attribute__((aligned(1024))) char smem[WAVES * 2 * SLOT];
 
-  const int nx = gridDim.x, ny = gridDim.y, heads = ny * gridDim.z;
-  const int hw = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
-  int x, head;
-  if (CAUSAL) {
-    wir::longest_first<true, 2048>(hw, nx, heads, x, head);
-  } else {
-    const int id = wir::remap_xcd(hw, nx * heads);
-    x = id % nx;
-    head = id / nx;
-  }
-  const int h = head % ny, b = head / ny, hkv = h / args.HR;
+  int x, h, b;
+  wir::split_program<CAUSAL, true>(x, h, b);
+  const int hkv = h / args.HR;
   const int row0 = x * ROWS, wave = wir::wave_id();
   const int keys = CAUSAL ? min(args.N, row0 + ROWS) : args.N;
   const int tiles = (keys + KT - 1) / KT;
@@ -154,19 +148,10 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
 
   // merge: partial O of wave w at part[w][row][col], then m and l of every row
   wir::wait_vm_barrier<0>();
-  __attribute__((address_space(3))) float* part = (__attribute__((address_space(3))) float*)wir::lds(smem);
-  __attribute__((address_space(3))) float* ml = part + WAVES * ROWS * PITCH;
+  lds_float* part = (lds_float*)wir::lds(smem);
+  lds_float* ml = part + WAVES * ROWS * PITCH;
+  wir::put_partial<D>(part, o, wave);
   const int lane = wir::lane_id(), lr = lane % 32, lh = lane / 32;
-#pragma unroll
-  for (int cb = 0; cb < D / 32; ++cb)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      f32x4 v;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = o.f[cb][0][4 * g + j];
-      *(__attribute__((address_space(3))) f32x4*)(part + (wave * ROWS + lr) * PITCH + cb * 32 + wir::ccol<32>(4 * g, lh)) =
-          v;
-    }
   if (lh == 0) {
     ml[wave * ROWS + lr] = m;
     ml[(WAVES + wave) * ROWS + lr] = l;
@@ -191,9 +176,9 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
     for (int w = 0; w < WAVES; ++w) {
       const float f = __builtin_amdgcn_exp2f(__builtin_fmaf(ml[w * ROWS + row], c, base));
       sum += f * ml[(WAVES + w) * ROWS + row];
-      const __attribute__((address_space(3))) float* p = part + (w * ROWS + row) * PITCH + ch * 8;
-      const f32x4 lo = *(const __attribute__((address_space(3))) f32x4*)p;
-      const f32x4 hi = *(const __attribute__((address_space(3))) f32x4*)(p + 4);
+      const lds_float* p = part + (w * ROWS + row) * PITCH + ch * 8;
+      const f32x4 lo = *(const lds_f32x4*)p;
+      const f32x4 hi = *(const lds_f32x4*)(p + 4);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         acc[j] += f * lo[j];
@@ -212,12 +197,7 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
 
 }  // namespace
 
-#define WIR_SPLITKV(D, KT, NAME, CAUSAL)                                                                   \
-  extern "C" __global__ void __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1))) \
-  NAME(const splitkv_args args) {                                                                          \
-    splitkv<D, KT, CAUSAL>(args);                                                                          \
-  }
-WIR_SPLITKV(64, 64, wir_attn_splitkv_d64, false)
-WIR_SPLITKV(64, 64, wir_attn_splitkv_d64_causal, true)
-WIR_SPLITKV(128, 32, wir_attn_splitkv_d128, false)
-WIR_SPLITKV(128, 32, wir_attn_splitkv_d128_causal, true)
+WIR_SPLIT_KERNEL(wir_attn_splitkv_d64, splitkv_args, (splitkv<64, 64, false>))
+WIR_SPLIT_KERNEL(wir_attn_splitkv_d64_causal, splitkv_args, (splitkv<64, 64, true>))
+WIR_SPLIT_KERNEL(wir_attn_splitkv_d128, splitkv_args, (splitkv<128, 32, false>))
+WIR_SPLIT_KERNEL(wir_attn_splitkv_d128_causal, splitkv_args, (splitkv<128, 32, true>))

@@ -298,7 +298,8 @@ TARGETS: Dict[str, dict] = {
     "gemm_128_splitk_k64_b7sw": {"dma_spread_whole": True},
     "gemm_128_splitk_k32_b14sw": {"dma_spread_whole": True},
 }
-# the products that api.gemm launches run ragged extents in the clamped body
+# the products that api.gemm launches, and the two that api.gemm_variant names without a K
+# (gemm_128_k64, gemm_128x32_k64), run ragged extents in the clamped body
 for _name in ("gemm_256_k64", "gemm_256x128", "gemm_128x256_k64", "gemm_128_k64", "gemm_128_k64_s3",
               "gemm_128x64_k64", "gemm_64x128_k64", "gemm_64_k64", "gemm_128x32_k64", "gemm_128_splitk_k64_b7"):
     TARGETS[_name] = {**TARGETS.get(_name, {}), "clamp_edges": True}
