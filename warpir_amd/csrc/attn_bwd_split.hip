@@ -47,7 +47,7 @@ struct Scale {
 template <int D>
 __device__ __forceinline__ void store_sum(const lds_float* part, const wir::gl<bf16>& g, int b, int h, int row0,
                                           float scale) {
-  const wir::RowStore out(g, b, h);
+  const wir::RowStore out(g, b, h, row0, D);
 #pragma unroll
   for (int it = 0; it < ROWS * (D / 8) / (WAVES * 64); ++it) {
     const int idx = it * WAVES * 64 + threadIdx.x;
@@ -68,7 +68,7 @@ __device__ __forceinline__ void store_sum(const lds_float* part, const wir::gl<b
     bf16x8 v;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (bf16)(acc[j] * scale);
-    out.put8(g, row0 + row, ch * 8, v);
+    out.put8(g, row, ch * 8, v);
   }
 }
 

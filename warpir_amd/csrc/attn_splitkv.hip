@@ -158,7 +158,7 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
   }
   wir::barrier();
 
-  const wir::RowStore out(args.O, b, h);
+  const wir::RowStore out(args.O, b, h, row0, D);
   float* lb = args.L.data + (long long)b * args.L.sb + (long long)h * args.L.sd;
   const int lse_rows = (unsigned)b < (unsigned)args.L.b && (unsigned)h < (unsigned)args.L.d ? args.L.r : 0;
 #pragma unroll
@@ -189,7 +189,7 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
     bf16x8 v;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = (bf16)(acc[j] * inv);
-    out.put8(args.O, row0 + row, ch * 8, v);
+    out.put8(args.O, row, ch * 8, v);
     if (ch == 0 && row0 + row < lse_rows)
       lb[(long long)(row0 + row) * args.L.sr] = (top * c + __builtin_amdgcn_logf(sum)) * kLn2;
   }
