@@ -103,3 +103,16 @@ def test_split_backward_special_values(gpu, taken, monkeypatch, where, bad, d, c
         # (where the fp32 reference is finite: its 0 * NaN of masked scores is NaN, theirs often not formed)
         both = g.isfinite() & e.isfinite()
         assert rel_err(g[both], e[both]) <= 1e-2
+
+
+@pytest.mark.parametrize("bsz,heads,seq,causal", [(32, 8, 64, True), (16, 8, 128, False), (8, 8, 256, True)])
+def test_many_short_heads_keep_the_tiled_kernels(gpu, taken, monkeypatch, bsz, heads, seq, causal):
+    """512 programs of a few tiles: two rounds of the split kernels are slower."""
+    split, real = [], api._attention_split_kv
+    monkeypatch.setattr(api, "_attention_split_kv", lambda *a: split.append(1) or real(*a))
+    monkeypatch.setattr(api, "_forward_plans", api.Plans("attention_forward"))
+    host, dev = _inputs(bsz, heads, seq, 64, causal)
+    got = api.attention_backward(*dev, causal=causal)
+    assert not taken and not split
+    for x, y in zip(got, attention_bwd_ref(*host, causal=causal)):
+        assert rel_err(x.cpu().float(), y) <= 1e-2

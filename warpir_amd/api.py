@@ -437,8 +437,9 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     elif hr > 1:
         raise ValueError(f"attention_forward: variant {variant} takes no grouped-query heads")
     packing = rec.pack(handle, args)
-    if planned and whole and _split_kv_fits(bsz * heads * (seq // 32), causal, packing[0]):
-        _attention_split_kv(packing, args, (bsz, heads, seq, d), hr, causal, rec)
+    shape = (bsz, heads, seq, d)
+    if planned and whole and _split_kv_fits(shape, causal, packing[0]):
+        _attention_split_kv(packing, args, shape, hr, causal, rec)
         return out, lse
     rec.kernel(handle, args, packing=packing)
     if rec:
@@ -446,16 +447,48 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     return out, lse
 
 
-def _split_kv_fits(programs: int, causal: bool, packed) -> bool:
-    """Whether the forward goes to the split-key kernel
-    (``attn_splitkv.hip``, 32 query rows per program, one program per CU).
-    It wins while its programs fit the CUs once, and causal ones, half of them
-    short, twice.  us, tiled -> split: B1 H8 S512 D64 10.3 -> 6.0 (128
-    programs), S1024 16.8 -> 9.2 (256), S1024 D128 26.6 -> 15.9; at 512
-    programs S2048 D64 30.0 -> 26.5 and D128 46.5 -> 48.5, causal 29.3 -> 18.5
-    and 41.1 -> 31.1; at 1024 B2 H8 S2048 D64 31.8 -> 49.9.  Its lane offsets
-    are 32-bit."""
-    return (0 < programs <= (512 if causal else 256)
+# The split attention kernels hold one program of 32 rows per CU at a time.  Up
+# to 256 programs they win at every length; up to 512, which start a second
+# round of them, where each has enough tiles to walk.  Shortest such S of causal
+# launches by programs (up to 320, 384, 448, 512): a causal launch's short
+# blocks fill the second round, so it pays earlier with fewer of them.  us,
+# tiled -> split, forward D64 H32 S320 9.0 -> 8.7, H44 S320 9.0 -> 9.9, H32 S512
+# 10.7 -> 10.1, H64 S256 7.6 -> 8.7; D128 H32 S320 12.3 -> 10.7, H27 S448 14.3 ->
+# 15.0, H24 S512 14.8 -> 13.7, H21 S768 19.5 -> 21.2, H18 S896 21.8 -> 20.6;
+# dQ + dK/dV D64 H32 S320 27.7 -> 24.0, H53 S192 22.3 -> 24.5, H37 S384 30.0 ->
+# 31.6, H32 S448 33.8 -> 27.9; D128 H32 S320 34.4 -> 31.1, H38 S320 36.1 -> 37.1,
+# H32 S384 37.2 -> 35.0, H37 S384 39.1 -> 43.0, H36 S448 42.4 -> 41.3.
+_SPLIT_CAUSAL_SEQ = {
+    ("forward", 64): (320, 320, 448, 448), ("forward", 128): (320, 512, 576, 896),
+    ("backward", 64): (320, 320, 448, 448), ("backward", 128): (320, 384, 448, 448),
+}
+
+
+def _split_wins(part: str, programs: int, seq: int, d: int, causal: bool) -> bool:
+    """Whether a launch of *programs* blocks of 32 rows is faster in the split
+    kernels (``attn_splitkv.hip``, ``attn_bwd_split.hip``) than in the tiled
+    ones.  us, tiled -> split, at 128 programs: forward B1 H8 S512 D64 10.3 -> 6.0,
+    dQ + dK/dV 32.2 -> 16.3.  Past 256 programs full launches take two whole
+    rounds: the forward never wins (S2048 D64 30.0 -> 26.5 but D128 46.5 ->
+    48.5), dQ + dK/dV at D64 from S640, or from S512 where the waves' tiles come
+    out even (H16 S512 32.4 -> 30.6, S576 34.7 -> 35.8, S640 37.6 -> 36.1), at D128
+    from S1024 (67.5 -> 66.4, S768 55.1 -> 56.3)."""
+    if not 0 < programs <= 512:
+        return False
+    if programs <= 256:
+        return True
+    if causal:
+        return seq >= _SPLIT_CAUSAL_SEQ[part, d][(programs - 257) // 64]
+    if part == "forward":
+        return False
+    return seq >= 1024 if d == 128 else seq >= 640 or seq == 512
+
+
+def _split_kv_fits(shape, causal: bool, packed) -> bool:
+    """Whether the forward on Q of *shape* goes to the split-key kernel; its
+    lane offsets are 32-bit."""
+    bsz, heads, seq, d = shape
+    return (_split_wins("forward", bsz * heads * (seq // 32), seq, d, causal)
             and 0 <= packed.K.sr < 1 << 23 and 0 <= packed.V.sr < 1 << 23)
 
 
@@ -559,7 +592,7 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     # (handle, arguments, views) of each launch in order
     launches = [(kernels.handle(f"mha_bwd_dq_prep_d{d}{sfx}"), dq_args, None),
                 (kernels.handle(f"mha_bwd_dkdv_d{d}{sfx}"), dkdv_args, views)]
-    if planned and whole and hr == 1 and _split_bwd_fits(bsz, heads, seq, q, k, v, do):
+    if planned and whole and hr == 1 and _split_bwd_fits((bsz, heads, seq, d), causal, q, k, v, do):
         _attention_bwd_split(launches, causal, rec, dvec)
         if rec:
             _backward_plans.add(1 if causal else 0, rec, dq, dk, dv)
@@ -577,14 +610,12 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     return dq, dk, dv
 
 
-def _split_bwd_fits(bsz: int, heads: int, seq: int, *loaded) -> bool:
-    """Whether the backward goes to the split kernels (``attn_bwd_split.hip``,
-    32 rows per program, one program per CU at a time).  dQ + dK/dV in us,
-    tiled -> split: B1 H8 S512 D64 14.9 + 17.5 -> 8.0 + 8.3 (128 programs), S1024
-    24.3 + 29.3 -> 11.3 + 12.5 (256); at 512 programs S2048 D64 43.5 + 53.1 ->
-    32.5 + 37.9, causal 42.3 + 64.4 -> 23.2 + 24.7, H16 S1024 D128 33.1 + 37.4 ->
-    33.5 + 35.6.  Their lane offsets are 32-bit."""
-    return 0 < bsz * heads * (seq // 32) <= 512 and all(0 <= t.stride(2) < 1 << 23 for t in loaded)
+def _split_bwd_fits(shape, causal: bool, *loaded) -> bool:
+    """Whether the backward goes to the split kernels; their lane offsets are
+    32-bit."""
+    bsz, heads, seq, d = shape
+    return (_split_wins("backward", bsz * heads * (seq // 32), seq, d, causal)
+            and all(0 <= t.stride(2) < 1 << 23 for t in loaded))
 
 
 _split_bwd_kernels: dict = {}
