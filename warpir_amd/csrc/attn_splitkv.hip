@@ -127,6 +127,9 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
   if (wave < tiles) load(wave, 0);
   if (wave + WAVES < tiles) load(wave + WAVES, 1);
 
+  const wir::RowStore out(args.O, b, h, row0, D);   // (here its arguments load under the first tiles')
+  float* lb = args.L.data + (long long)b * args.L.sb + (long long)h * args.L.sd;
+  const int lse_rows = (unsigned)b < (unsigned)args.L.b && (unsigned)h < (unsigned)args.L.d ? args.L.r : 0;
   wir::RTile<32, 32, D> o;
   wir::fill(o, 0.f);
   float m = -__builtin_inff(), l = 0.f;
@@ -158,9 +161,6 @@ __device__ __forceinline__ void splitkv(const splitkv_args& args) {
   }
   wir::barrier();
 
-  const wir::RowStore out(args.O, b, h, row0, D);
-  float* lb = args.L.data + (long long)b * args.L.sb + (long long)h * args.L.sd;
-  const int lse_rows = (unsigned)b < (unsigned)args.L.b && (unsigned)h < (unsigned)args.L.d ? args.L.r : 0;
 #pragma unroll
   for (int it = 0; it < ROWS * (D / 8) / (WAVES * 64); ++it) {
     const int idx = it * WAVES * 64 + threadIdx.x;
