@@ -59,12 +59,13 @@ __device__ __forceinline__ void put_partial(lds_float* part, const RTile<32, 32,
 // and rows that are not 16-byte aligned (the host checks the row stride, not
 // the batch and head strides) take single stores.  `whole`, the same for all
 // lanes, skips the checks.  Forward, us, stores without bounds / a test per
-// chunk / this: B1 H8 S512 D64 5.79 / 5.99 / 5.87, D128 9.3 / - / 9.5.
+// chunk / this: B1 H8 S512 D64 5.79 / 5.99 / 5.87, D128 9.3 / - / 9.45.
 struct RowStore {
   bf16* base;
   int row0;
   bool in, whole;
 
+  __device__ __forceinline__ RowStore() {}
   __device__ __forceinline__ RowStore(const gl<bf16>& g, int b, int d, int row0_, int cols) : row0(row0_) {
     base = g.data + (long long)b * g.sb + (long long)d * g.sd;
     in = (unsigned)b < (unsigned)g.b && (unsigned)d < (unsigned)g.d;
