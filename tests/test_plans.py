@@ -33,5 +33,6 @@ def test_cpu_calls_record_nothing():
     for loaded in (False, True):
         if loaded:
             plans.native()
-        done, rec = plans.Plans("x").run(0, t, t.clone())
-        assert not done and rec is plans.NO_RECORDING and not rec and rec.alloc(t) is t
+        table = plans.Plans("x")
+        rec = table.recording(table.run(0, t, t.clone()), t)
+        assert rec is plans.NO_RECORDING and not rec and rec.alloc(t) is t

@@ -16,7 +16,7 @@ import math
 from typing import Optional, Tuple
 
 from warpir_amd import kernels
-from warpir_amd.plans import NO_RECORDING, Plans, Recording
+from warpir_amd.plans import Plans, Recording
 from warpir_amd.runtime import GL, RawKernel
 
 # Plans of the calls below, by flags: gemm 0; attention_forward and
@@ -330,17 +330,18 @@ def gemm(a, b, out=None, variant: Optional[str] = None, workspace=None):
     """
     import torch
 
-    rec = NO_RECORDING
+    done = None
     if variant is None and workspace is None:
-        done, rec = _gemm_plans.run(0, a, b, out)
-        if done:
-            return rec
+        done = _gemm_plans.run(0, a, b, out)
+        if done is not None and done is not False:
+            return done
     if a.dim() != 2 or b.dim() != 2 or a.shape[1] != b.shape[0]:
         raise ValueError(f"gemm: shapes {tuple(a.shape)} @ {tuple(b.shape)} do not chain")
     m, k = a.shape
     n = b.shape[1]
     if k % 8 or n % 8:
         raise ValueError("gemm: K and N must be multiples of 8 (16-byte rows)")
+    rec = _gemm_plans.recording(done, a, b, out)
     given = out is not None
     if not given:
         out = rec.alloc(torch.empty(m, n, dtype=torch.bfloat16, device=a.device))
@@ -402,11 +403,11 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     import torch
 
     planned = variant is None and type(causal) in (bool, int) and 0 <= causal <= 1   # others are refused below
-    rec = NO_RECORDING
+    done = None
     if planned:
-        done, rec = _forward_plans.run(1 if causal else 0, q, k, v, out, lse)
-        if done:
-            return rec
+        done = _forward_plans.run(1 if causal else 0, q, k, v, out, lse)
+        if done is not None and done is not False:
+            return done
     bsz, heads, seq, d = q.shape
     hr = _head_ratio("attention_forward", q, k, v)
     if variant is None:
@@ -425,6 +426,7 @@ def attention_forward(q, k, v, causal: bool = False, out=None, lse=None,
     kv_tile = _kv_tile(variant)
     if seq % kv_tile:
         raise ValueError(f"attention_forward: S={seq} must be a multiple of the KV tile {kv_tile}")
+    rec = _forward_plans.recording(done, q, k, v, out, lse)
     # (the tiled kernels' grid covers destinations of other shapes: what does not fit is dropped)
     whole = (out is None or out.shape == q.shape) and (lse is None or lse.shape == (bsz, heads, seq))
     if out is None:
@@ -552,11 +554,11 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
     import torch
 
     planned = workspace is None
-    rec = NO_RECORDING
+    done = None
     if planned:
-        done, rec = _backward_plans.run(1 if causal else 0, q, k, v, o, lse, do, dq, dk, dv, dvec)
-        if done:
-            return rec
+        done = _backward_plans.run(1 if causal else 0, q, k, v, o, lse, do, dq, dk, dv, dvec)
+        if done is not None and done is not False:
+            return done
     if q.dim() != 4 or not (q.shape == o.shape == do.shape):
         raise ValueError("attention_backward: q, o, do must share one [B, H, S, D] shape")
     hr = _head_ratio("attention_backward", q, k, v)
@@ -565,6 +567,7 @@ def attention_backward(q, k, v, o, lse, do, dq=None, dk=None, dv=None, dvec=None
         raise ValueError(f"attention_backward: D must be 64 or 128 and S a multiple of 64 (got D={d}, S={seq})")
     if tuple(lse.shape) != (bsz, heads, seq) or lse.dtype != torch.float32:
         raise ValueError("attention_backward: lse must be fp32 [B, H, S]")
+    rec = _backward_plans.recording(done, q, k, v, o, lse, do, dq, dk, dv, dvec)
     whole = (all(g is None or g.shape == q.shape for g in (dq, dk, dv))   # as in the forward
              and (dvec is None or dvec.shape == lse.shape))
     dq = rec.alloc(torch.empty_like(q)) if dq is None else dq

@@ -114,30 +114,32 @@ class Plans:
         self._table = None
 
     def run(self, flags: int, *tensors):
-        """(whether the call ran by its plan, its results; or the recording of
-        a call that has none: ``NO_RECORDING`` where none can be kept, so that
-        nothing is packed for it in vain).  us, without plans / recording in
-        vain / now: gemm under ``torch.set_default_device`` 28 / 68 / 28,
-        the tiled backward 123 / 289 / 109."""
+        """The call's results by its plan; False where it has none and can
+        leave one, None where it can not."""
         table = self._table
         if table is None:
             if _native is None and not getattr(tensors[0], "is_cuda", False):
-                return False, NO_RECORDING
+                return None
             mod = native()
             with _lock:
                 if self._table is None:
                     self._table = mod.table()
                 table = self._table
         r = _native.run(table, flags, *tensors)
-        if r is None:
-            return False, NO_RECORDING
-        if r is False:
-            return False, Recording(*tensors)
         if type(r) is int:
             from warpir_amd.runtime import check
 
             check(r, self.what)
-        return True, r
+        return r
+
+    @staticmethod
+    def recording(missed, *inputs):
+        """A recording for a call whose ``run`` gave *missed*: ``NO_RECORDING``
+        for None, so that nothing is packed for a plan in vain.  us, without
+        plans / recording in vain / now: gemm under
+        ``torch.set_default_device`` 28 / 68 / 28, the tiled backward 123 / 289
+        / 109."""
+        return Recording(*inputs) if missed is False else NO_RECORDING
 
     def add(self, flags: int, rec: Recording, *results) -> None:
         """Keep the plan of a call that has just run."""
