@@ -236,6 +236,8 @@ def gemm_split_k(a, b, out=None, splits: Optional[int] = None, workspace=None, v
                          f"{out.dtype} {tuple(out.shape)} with strides {tuple(out.stride())}")
     if out.device != a.device:
         raise ValueError("gemm_split_k: out must be on the operands' device")
+    if not all(t.data_ptr() for t in (a, b, out) if t.numel()):   # (of a null workspace the library says so)
+        raise ValueError("gemm_split_k: a tensor has no memory (a fake or meta tensor)")
     if workspace is None:
         workspace = torch.empty(splits * m * n, dtype=torch.float32, device=a.device)
     if workspace.numel() < splits * m * n or workspace.dtype != torch.float32:
@@ -663,6 +665,8 @@ def _group_reduce(partials, out, splits: int):
         raise ValueError("attention_backward: dk / dv must be contiguous bf16")
     if out.numel() == 0:
         return None
+    if out.device != partials.device or not out.data_ptr():
+        raise ValueError("attention_backward: dk / dv must be in the memory of the operands' GPU")
     n = out.shape[-2] * out.shape[-1]
     groups = out.numel() // n
     if n % 8 or partials.numel() != groups * splits * n:

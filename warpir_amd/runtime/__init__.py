@@ -336,6 +336,8 @@ class KernelHandle:
                     if x.data_ptr() % 16 or (strides[2] * esz) % 16 or (shape[3] * esz) % 16:
                         raise ValueError(f"{v.name}: rows must be 16-byte aligned and a multiple of 16 bytes "
                                          "(the tile-load granule)")
+                if x.numel() and not x.data_ptr():   # a kernel would follow the null pointer
+                    raise ValueError(f"{v.name}: has no memory (a fake or meta tensor)")
                 for dim in shape:
                     if dim >= 2 ** 31:
                         raise ValueError(f"{v.name}: dimension {dim} does not fit in int32")
