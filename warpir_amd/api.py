@@ -230,14 +230,12 @@ def gemm_split_k(a, b, out=None, splits: Optional[int] = None, workspace=None, v
         raise TypeError("gemm_split_k: a and b must be bf16")
     if out is None:
         out = torch.empty(m, n, dtype=torch.bfloat16, device=a.device)
-    # the reduction writes M * N bf16 values flat from out's first element
+    # the reduction writes M * N bf16 values flat from out's first element (the library refuses null pointers)
     if tuple(out.shape) != (m, n) or out.dtype != torch.bfloat16 or not out.is_contiguous():
         raise ValueError(f"gemm_split_k: out must be a contiguous bf16 [{m}, {n}] tensor, got "
                          f"{out.dtype} {tuple(out.shape)} with strides {tuple(out.stride())}")
     if out.device != a.device:
         raise ValueError("gemm_split_k: out must be on the operands' device")
-    if not all(t.data_ptr() for t in (a, b, out) if t.numel()):   # (of a null workspace the library says so)
-        raise ValueError("gemm_split_k: a tensor has no memory (a fake or meta tensor)")
     if workspace is None:
         workspace = torch.empty(splits * m * n, dtype=torch.float32, device=a.device)
     if workspace.numel() < splits * m * n or workspace.dtype != torch.float32:
